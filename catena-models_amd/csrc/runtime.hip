@@ -24,6 +24,7 @@
 #include "mega.h"
 #include "dense_step.h"
 #include "prefill.h"
+#include "bgemm.h"
 #include "mfma.h"
 #include "gguf.h"
 #include "batch.h"
@@ -351,6 +352,7 @@ struct cq35_model {
   cq35_config cfg;
   Dims d;
   int device = 0;
+  int cus = 256;              // compute units
   std::vector<void*> w;       // device pointers in weight ABI order
   std::vector<void*> owned;   // allocations to free
   float* freq = nullptr;      // F32 theta^(-2i/R) (src/catena.rs:185-232)
@@ -362,6 +364,7 @@ struct cq35_model {
 namespace {
 
 int finish_model(cq35_model* m) {
+  HIP_TRY(hipDeviceGetAttribute(&m->cus, hipDeviceAttributeMultiprocessorCount, m->device));
   const int half = (int)(m->cfg.rope_dim / 2);
   std::vector<float> f(std::max(half, 1));
   for (int i = 0; i < half; ++i)
@@ -778,6 +781,7 @@ struct cq35_session {
   float *pf_part = nullptr, *pf_spart = nullptr;  // matrix-core experts: routed / shared down sums
   int *pf_eoff = nullptr, *pf_order = nullptr;    // matrix-core experts: buckets
   int* pf_ids = nullptr;
+  uint32_t* pf_ranges = nullptr;  // k_bgemm: magnitude ranges of a launch's weight and token tiles
   int pf_attn_tokens = 0;  // tokens per staged-attention launch (scratch rows)
   int pf_rows = 0;         // token rows of the chunk buffers
   int matrix = 0;          // CQ35_MATRIX_* components of multi-token calls on MFMA
@@ -1433,6 +1437,48 @@ const char* prefill_unsupported(const cq35_model& m) {
   return nullptr;
 }
 
+// The exact projections of n token rows on the matrix cores (k_bgemm, then
+// k_bgemm_fix): widths of whole 128-byte lines, eight tokens or more. Below,
+// k_bproject: a tile's sixteen columns would be mostly empty (four 2B layers,
+// whole call, at 5 / 8 tokens: 871 / 1073 us against 916 / 923 here).
+bool bgemm_ok(int n, int64_t cols) { return cols % 64 == 0 && n >= kBTokens; }
+
+template <int kMode, int TT, int RT>
+void bgemm_launch(Launcher& L, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2,
+                  const uint16_t* res, uint32_t* ranges) {
+  using T = BGemmTile<TT, RT>;
+  const int per = bgemm_rows<kMode, RT>();
+  const int tr = (int)((seg_rows(seg) + per - 1) / per), tt = (n + T::kTokens - 1) / T::kTokens;
+  const int grid = std::min((tr + 7) / 8 * tt, std::max(L.s->model->cus / 8, 1) * T::kBlocksPerCu) * 8;
+  L(KC_PREFILL_PROJECT, k_bgemm<kMode, TT, RT>, dim3((unsigned)grid), dim3(kEThreads), T::kLds, x, n, cols, seg, w2, res,
+    ranges);
+  L(KC_PREFILL_PROJECT, k_bgemm_fix<kMode, TT, RT>, dim3((unsigned)((tr * tt + kBlock - 1) / kBlock)), dim3(kBlock), 0, x,
+    n, cols, seg, w2, res, (const uint32_t*)ranges);
+}
+
+// Few tokens: 16 x 16 tiles, two blocks per CU (more tiles to spread and one
+// block's barriers behind the other's products); many: 48 x 16, fewer
+// operands per product. 12352 rows x 2048 at 37 / 256 / 768 tokens: 59 / 240 /
+// 683 us against 69 / 262 / 653; the gate mode, with two row halves per tile,
+// turns earlier (6144 x 2048 twice at 16 / 128: 32 / 147 against 50 / 135).
+template <int kMode>
+void bgemm(Launcher& L, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2, const uint16_t* res,
+           uint32_t* ranges) {
+  if (n <= (kMode == kBGate ? 32 : 256)) bgemm_launch<kMode, 1, 1>(L, x, n, cols, seg, w2, res, ranges);
+  else bgemm_launch<kMode, 3, 1>(L, x, n, cols, seg, w2, res, ranges);
+}
+
+hipError_t bgemm_lds_optin() {
+  const std::pair<const void*, size_t> f[] = {
+      {(const void*)k_bgemm<kBPlain, 1, 1>, BGemmTile<1, 1>::kLds}, {(const void*)k_bgemm<kBPlain, 3, 1>, BGemmTile<3, 1>::kLds},
+      {(const void*)k_bgemm<kBResidual, 1, 1>, BGemmTile<1, 1>::kLds}, {(const void*)k_bgemm<kBResidual, 3, 1>, BGemmTile<3, 1>::kLds},
+      {(const void*)k_bgemm<kBGate, 1, 1>, BGemmTile<1, 1>::kLds}, {(const void*)k_bgemm<kBGate, 3, 1>, BGemmTile<3, 1>::kLds}};
+  hipError_t e = hipSuccess;
+  for (const auto& k : f)
+    if (e == hipSuccess) e = hipFuncSetAttribute(k.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.second);
+  return e;
+}
+
 // Chunk buffers of the batched prefill: kBChunk token rows, or kMChunk when
 // the session has matrix-core components selected at its first multi-token
 // call (their expert weights are then streamed once per kMChunk tokens).
@@ -1456,6 +1502,8 @@ int setup_prefill(cq35_session* s) {
   check(dalloc(s, &s->pf_g, m * d.VS));                       // gated
   check(dalloc(s, &s->pf_act, m * std::max(d.I, d.K * d.I + d.SI)));
   check(dalloc(s, &s->pf_rope, m * std::max<int64_t>(d.R, 2)));
+  check(dalloc(s, &s->pf_ranges, std::max({d.QKV + d.VS + 2 * VH, 2 * d.QS + 2 * d.KVS, d.H, d.I}) + m + 2 * 8 * kEWaves));
+  if (!rc && bgemm_lds_optin() != hipSuccess) rc = fail(CQ35_EDEVICE, "projection kernels' LDS");
   if (c.moe) {
     check(dalloc(s, &s->pf_logits, m * (d.E + 1)));
     check(dalloc(s, &s->pf_ids, m * d.K));
@@ -1517,6 +1565,10 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
           rows_n, cols, seg, (const uint16_t*)nullptr, (const uint16_t*)nullptr);
         return true;
       }
+      if (!mp && bgemm_ok(rows_n, cols)) {
+        bgemm<kBPlain>(L, x, rows_n, cols, seg, nullptr, nullptr, s->pf_ranges);
+        return true;
+      }
       return false;
     };
     auto project = [&](const uint16_t* x, int cols, const void* w, int rows, uint16_t* out) {
@@ -1540,6 +1592,8 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
       else if (mp && cols % 16 == 0)
         L(KC_PREFILL_PROJECT, k_mproject<kBResidual>, mgrid(H, cols), dim3(64 * kMWaves), 0, x, rows_n, cols,
           (const uint16_t*)w, (const uint16_t*)nullptr, H, res, out);
+      else if (!mp && bgemm_ok(rows_n, cols))
+        bgemm<kBResidual>(L, x, rows_n, cols, segments({{w, {out, H}}}), nullptr, res, s->pf_ranges);
       else
         L(KC_PREFILL_PROJECT, k_bproject<kBResidual>,
           dim3((unsigned)((H + bproject_rows<kBResidual>() - 1) / bproject_rows<kBResidual>()), tiles), dim3(kBlock), 0, x,
@@ -1749,6 +1803,9 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
             L(KC_PREFILL_PROJECT, k_mproject<kBGate>, mgrid((int)d.I, H), dim3(64 * kMWaves), 0,
               (const uint16_t*)s->pf_x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
               (int)d.I, (const uint16_t*)nullptr, s->pf_act);
+        else if (!mp && bgemm_ok(rows_n, H))
+          bgemm<kBGate>(L, s->pf_x, rows_n, H, segments({{W(ffn), {s->pf_act, d.I}}}), (const uint16_t*)W(ffn + 1),
+                        nullptr, s->pf_ranges);
         else
           L(KC_PREFILL_PROJECT, k_bproject<kBGate>, dim3((unsigned)d.I, tiles), dim3(kBlock), 0,
             (const uint16_t*)s->pf_x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
