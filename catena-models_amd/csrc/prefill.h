@@ -172,53 +172,128 @@ __global__ __launch_bounds__(kBlock) void k_bnorm(const uint16_t* __restrict__ x
 // Four-tap convolution of every token of the chunk, then the per-head L2
 // norm of the Q and K heads (batch.prepare, batch_prepare.hex:3-158): the tap
 // at position p < `first` reads the cache history slot p % 3 (still holding
-// the rows before this chunk), later taps read the chunk's own rows. Block
-// (KD-channel chunk, token).
+// the rows before this chunk), later taps read the chunk's own rows.
+//
+// Block (KD channels, TB tokens), a thread two channels of TB / 4 consecutive
+// tokens: each row is read once per thread (and three rows before its first),
+// the serial sum of squares of a token's head runs on a lane of its own, all
+// tokens at once (one block per token left 255 threads waiting for it: 1024
+// tokens of a 35B layer 70 us, now 30). TB 8 for short calls, where a thread's
+// tokens in turn would be the time (37 tokens: 6 us, 10 at TB 32).
+constexpr int kPrepareTokens = 32, kPrepareFew = 8;
+
+template <int KD, int TB>
 __global__ __launch_bounds__(kBlock) void k_bprepare(
     const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ cache, int64_t conv_base,
-    const uint64_t* __restrict__ params, int first, const float* __restrict__ conv_w, int qkv_size,
-    int key_dim, int key_heads, uint16_t* __restrict__ conv_out, uint16_t* __restrict__ q_out,
+    const uint64_t* __restrict__ params, int first, int m, const float* __restrict__ conv_w, int qkv_size,
+    int key_heads, uint16_t* __restrict__ conv_out, uint16_t* __restrict__ q_out,
     uint16_t* __restrict__ k_out) {
-  __shared__ float squares[256];
-  __shared__ float total;
-  const int t = blockIdx.y;
+  constexpr int kPairs = KD / 2, kGroups = kBlock / kPairs, kEach = TB / kGroups;
+  static_assert(kBlock % kPairs == 0 && TB % kGroups == 0, "channel pairs");
+  __shared__ float squares[TB][KD + 1];
+  __shared__ float total[TB];
   const int64_t begin = (int64_t)params[0] + first;  // position of the chunk's row 0
-  const int64_t position = begin + t;
-  const int chunk = blockIdx.x, tid = threadIdx.x;
-  const int ch = chunk * key_dim + tid;
-  const bool active = tid < key_dim && ch < qkv_size;
-  const int key_size = key_heads * key_dim;
-  float value = 0.0f;
-  if (active) {
-    float taps[3];
+  const int chunk = blockIdx.x, pair = threadIdx.x % kPairs, group = threadIdx.x / kPairs;
+  const int t0 = blockIdx.y * TB + group * kEach;
+  const int ch = chunk * KD + 2 * pair;
+  const bool active = ch < qkv_size;
+  const int key_size = key_heads * KD;
+  const bool heads = chunk < 2 * key_heads;  // value heads: convolution only
+  auto row = [&](int t) -> uint32_t {        // the chunk's row t, or the history before it
+    const int64_t p = begin + t;
+    if (p < 0) return 0u;
+    const uint16_t* r = t < 0 ? cache + conv_base + (p % 3) * qkv_size : qkv + (size_t)t * qkv_size;
+    return *reinterpret_cast<const uint32_t*>(r + ch);
+  };
+  float value[kEach][2];
+  if (active && t0 < m) {
+    const f32x4 w0 = reinterpret_cast<const f32x4*>(conv_w)[ch], w1 = reinterpret_cast<const f32x4*>(conv_w)[ch + 1];
+    uint32_t in[kEach + 3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int64_t p = position - 3 + k;
-      float input = 0.0f;
-      if (p >= 0)
-        input = p < begin ? bf2f(cache[conv_base + (p % 3) * qkv_size + ch])
-                          : bf2f(qkv[(size_t)(p - begin) * qkv_size + ch]);
-      taps[k] = input * conv_w[(size_t)ch * 4 + k];
+    for (int i = 0; i < kEach + 3; ++i) in[i] = row(min(t0 - 3 + i, m - 1));
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+      auto conv = [&](auto half, const f32x4& w) {
+        auto x = [&](int k) { return decltype(half)::value ? hi2f(in[i + k]) : lo2f(in[i + k]); };
+        const float sum = (x(0) * w[0] + x(2) * w[2]) + (x(1) * w[1] + x(3) * w[3]);
+        return f2bf(silu(rbf(sum)));
+      };
+      const uint16_t lo = conv(std::false_type{}, w0), hi = conv(std::true_type{}, w1);
+      if (t0 + i < m) *reinterpret_cast<uint32_t*>(conv_out + (size_t)(t0 + i) * qkv_size + ch) = pack_bf(lo, hi);
+      value[i][0] = bf2f(lo);
+      value[i][1] = bf2f(hi);
+      if (heads) {
+        squares[group * kEach + i][2 * pair] = value[i][0] * value[i][0];
+        squares[group * kEach + i][2 * pair + 1] = value[i][1] * value[i][1];
+      }
     }
-    const float tap3 = bf2f(qkv[(size_t)t * qkv_size + ch]) * conv_w[(size_t)ch * 4 + 3];
-    const float sum = (taps[0] + taps[2]) + (taps[1] + tap3);
-    const uint16_t result = f2bf(silu(rbf(sum)));
-    conv_out[(size_t)t * qkv_size + ch] = result;
-    value = bf2f(result);
   }
-  if (chunk >= 2 * key_heads) return;  // value heads: convolution only
-  if (tid < key_dim) squares[tid] = value * value;
+  if (!heads) return;  // uniform
   __syncthreads();
-  if (tid == 0) {
+  if (threadIdx.x < TB && blockIdx.y * TB + (int)threadIdx.x < m) {
     float s = 0.0f;
-    for (int i = 0; i < key_dim; ++i) s += squares[i];
-    total = s;
+#pragma unroll 16
+    for (int i = 0; i < KD; ++i) s += squares[threadIdx.x][i];
+    total[threadIdx.x] = nsqrt(s + bitsf(0x358637bdu));
   }
   __syncthreads();
-  if (tid < key_dim) {
-    const float norm = nsqrt(total + bitsf(0x358637bdu));
-    uint16_t* dst = (chunk < key_heads ? q_out : k_out) + (size_t)t * key_size;
-    dst[(chunk % key_heads) * key_dim + tid] = f2bf(value / norm);
+  uint16_t* dst = (chunk < key_heads ? q_out : k_out) + (chunk % key_heads) * KD + 2 * pair;
+#pragma unroll
+  for (int i = 0; i < kEach; ++i) {
+    if (t0 + i >= m) break;
+    const float norm = total[group * kEach + i];
+    *reinterpret_cast<uint32_t*>(dst + (size_t)(t0 + i) * key_size) =
+        pack_bf(f2bf(value[i][0] / norm), f2bf(value[i][1] / norm));
+  }
+}
+
+// k_gated_norm (layers.h) over the chunk's (token, head) rows of value_dim
+// contiguous values: `per` (at most kGatedRows) rows per block, a row's serial
+// sum of squares on a lane of its own, the rest eight values at a time. One
+// block per row left 255 threads waiting for that sum: 1024 tokens of a 35B
+// layer 34 us, now 16. value_dim % 8 == 0, at most 256.
+constexpr int kGatedRows = 32;
+inline size_t bgated_lds_bytes(int value_dim) { return (size_t)kGatedRows * (value_dim + 2) * 4; }
+
+__global__ __launch_bounds__(kBlock) void k_bgated_norm(const uint16_t* __restrict__ core,
+                                                        const uint16_t* __restrict__ z, const float* __restrict__ w,
+                                                        int rows, int per, int value_dim, float eps,
+                                                        uint16_t* __restrict__ out) {
+  extern __shared__ float bgn_lds[];
+  float* squares = bgn_lds;  // [row][value_dim + 1]
+  float* rms = bgn_lds + kGatedRows * (value_dim + 1);
+  const int r0 = blockIdx.x * per, quads = value_dim >> 3;
+  const int count = min(per, rows - r0) * quads;
+  const size_t base = (size_t)r0 * quads;
+  for (int i = threadIdx.x; i < count; i += kBlock) {
+    const u32x4 v = ldq(core, base + i);
+    float* s = squares + (i / quads) * (value_dim + 1) + 8 * (i % quads);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[2 * e] = lo2f(v[e]) * lo2f(v[e]);
+      s[2 * e + 1] = hi2f(v[e]) * hi2f(v[e]);
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < min(per, rows - r0)) {
+    float s = 0.0f;
+#pragma unroll 8
+    for (int i = 0; i < value_dim; ++i) s += squares[threadIdx.x * (value_dim + 1) + i];
+    rms[threadIdx.x] = nsqrt(s / (float)value_dim + eps);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < count; i += kBlock) {
+    const u32x4 v = ldq(core, base + i), zq = ldq(z, base + i);
+    const float d = rms[i / quads];
+    const f32x4* wq = reinterpret_cast<const f32x4*>(w) + 2 * (i % quads);
+    const f32x4 wl = wq[0], wh = wq[1];
+    u32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = e < 2 ? wl[2 * e] : wh[2 * e - 4], b = e < 2 ? wl[2 * e + 1] : wh[2 * e - 3];
+      y[e] = pack_bf(f2bf((lo2f(v[e]) / d * a) * silu(lo2f(zq[e]))), f2bf((hi2f(v[e]) / d * b) * silu(hi2f(zq[e]))));
+    }
+    reinterpret_cast<u32x4*>(out)[base + i] = y;
   }
 }
 
@@ -239,20 +314,45 @@ __global__ __launch_bounds__(kBlock) void k_bhistory(const uint16_t* __restrict_
   }
 }
 
+// Sum over the 32 lanes of each half wave, the total in every lane: the
+// halving tree's operands (strides 16 ... 1; a lane past the first s of a
+// level adds the same two values the other way round).
+__device__ __forceinline__ float sum32_everywhere(float v) {
+  const int b = __builtin_bit_cast(int, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);  // a half's first row, its second
+  v = __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+  auto turned = [](float x, auto ror) {
+    const int i = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, 0x120 + decltype(ror)::value, 0xf, 0xf, true));
+  };
+  v += turned(v, std::integral_constant<int, 8>{});
+  v += turned(v, std::integral_constant<int, 4>{});
+  v += turned(v, std::integral_constant<int, 2>{});
+  v += turned(v, std::integral_constant<int, 1>{});
+  return v;
+}
+
 // DeltaNet scan over the chunk's tokens with the F32 state in registers
 // (batch.scan, batch_scan.hex:1-200): per token exactly the single-step
 // arithmetic of k_delta (32 lanes per value channel, lane l owns key elements
-// l, l+32, ...; serial from 0.0, 32-wide halving tree), 8 channels of one
-// head per block. Requires key_dim <= 256 and value_dim % 8 == 0.
+// l, l+32, ...; serial from 0.0, 32-wide halving tree), 8 channels of one head
+// per block. Requires key_dim <= 256 and value_dim % 8 == 0.
 //
-// The serial chain reads only LDS: per stage of kScanTokens tokens the
-// block first stages the head's k and q rows (lane-major, lane l's elements
-// l + 32 j contiguous), its channels' values, and every token's decay and
-// rate (computed in parallel: they do not depend on the state).
-constexpr int kScanTokens = 64;
+// Bound: instruction issue of a token's serial chain (two sums over 32
+// reference lanes, the state update between them). The chain holds nothing
+// else: per stage of kScanTokens tokens the block first stages the head's k
+// and q rows widened to F32, its channels' values, and every token's decay
+// and rate (the next stage's rows are requested before the chain starts); a
+// token's values are read from LDS a token ahead; the sums leave their total
+// in every lane; lane t keeps token t's output, and scale, rounding and store
+// run once per stage: 67 vector instructions a token. 1024 tokens of a 35B
+// layer take 225 us (355 with BF16 rows widened and the totals broadcast
+// inside the chain; 16 lanes per channel, a quarter fewer instructions but one
+// wave per SIMD: 218).
+constexpr int kScanTokens = 32;
 
 __host__ __device__ constexpr size_t bscan_lds_bytes(int key_dim) {
-  return (size_t)kScanTokens * key_dim * 2 * 2 + (size_t)kScanTokens * (2 + 8) * 4;
+  return (size_t)kScanTokens * key_dim * 2 * 4 + (size_t)kScanTokens * 8 + (size_t)kScanTokens * 8 * (4 + 2);
 }
 
 template <int KJ>  // key elements per lane: key_dim / 32
@@ -260,90 +360,119 @@ __global__ __launch_bounds__(kBlock) void k_bscan(
     const uint16_t* __restrict__ conv, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ alpha,
     const uint16_t* __restrict__ beta, const float* __restrict__ dt, const float* __restrict__ a,
-    float* __restrict__ state, int m, int value_size, int value_dim, int value_heads, int key_dim,
-    int key_heads, int qkv_size, float scale, uint16_t* __restrict__ out) {
+    float* __restrict__ state, int m, int value_size, int value_dim, int value_heads, int key_heads, int qkv_size,
+    float scale, uint16_t* __restrict__ out) {
+  constexpr int key_dim = 32 * KJ, quads = key_dim / 8;
+  constexpr int CH = kBlock / 32;  // channels
+  constexpr int kRows = kScanTokens * quads / kBlock;  // quads of k and of q per thread and stage
+  static_assert(kScanTokens == 32 && kScanTokens * CH == kBlock, "a token per lane, a value per thread");
   extern __shared__ __align__(16) unsigned char scan_lds[];
-  uint16_t* sk = reinterpret_cast<uint16_t*>(scan_lds);
-  uint16_t* sq = sk + kScanTokens * key_dim;
-  float* sdecay = reinterpret_cast<float*>(sq + kScanTokens * key_dim);
-  float* srate = sdecay + kScanTokens;
-  float* sval = srate + kScanTokens;  // [token][8]
-  const int c0 = blockIdx.x * 8;
-  const int ch = threadIdx.x >> 5;
+  float* sk = reinterpret_cast<float*>(scan_lds);
+  float* sq = sk + kScanTokens * key_dim;
+  float2* sgate = reinterpret_cast<float2*>(sq + kScanTokens * key_dim);  // decay, rate
+  float* sval = reinterpret_cast<float*>(sgate + kScanTokens);            // [token][CH]
+  uint16_t* sout = reinterpret_cast<uint16_t*>(sval + kScanTokens * CH);  // [token][CH]
+  const int c0 = blockIdx.x * CH;
+  const int ch = threadIdx.x / 32;
   const int c = c0 + ch;
-  const int lane = threadIdx.x & 31, half = (threadIdx.x >> 5) & 1;
-  const bool valid = c < value_size;
-  const int cc = valid ? c : 0;
-  const int head = min(c0, value_size - 1) / value_dim;
+  const int lane = threadIdx.x % 32;
+  const int head = c0 / value_dim;
   const int kbase = (head % key_heads) * key_dim;
   const int key_size = key_heads * key_dim;
-  constexpr int kj = KJ;
   const float dth = dt[head], ah = a[head];
   float s[KJ];
 #pragma unroll
-  for (int j = 0; j < KJ; ++j) s[j] = state[(size_t)cc * key_dim + lane + 32 * j];
+  for (int j = 0; j < KJ; ++j) s[j] = state[(size_t)c * key_dim + lane + 32 * j];
+  u32x4 kq4[kRows > 0 ? kRows : 1], qq4[kRows > 0 ? kRows : 1];
+  uint16_t val, al, be;
+  // a stage's rows into registers (rows past the last repeat it)
+  auto request = [&](int t0) {
+#pragma unroll
+    for (int r = 0; r < (kRows > 0 ? kRows : 1); ++r) {
+      const int idx = threadIdx.x + kBlock * r;
+      const int t = min(t0 + min(idx / quads, kScanTokens - 1), m - 1);
+      const size_t src = (size_t)t * key_size + kbase + 8 * (idx % quads);
+      kq4[r] = *reinterpret_cast<const u32x4*>(k + src);
+      qq4[r] = *reinterpret_cast<const u32x4*>(q + src);
+    }
+    val = conv[(size_t)min(t0 + (int)threadIdx.x / CH, m - 1) * qkv_size + 2 * key_size + c0 + threadIdx.x % CH];
+    const int t = min(t0 + lane, m - 1);
+    al = alpha[(size_t)t * value_heads + head];
+    be = beta[(size_t)t * value_heads + head];
+  };
+  auto place = [&]() {
+#pragma unroll
+    for (int r = 0; r < (kRows > 0 ? kRows : 1); ++r) {
+      const int idx = threadIdx.x + kBlock * r;
+      if (idx >= kScanTokens * quads) continue;
+      auto widen = [&](float* to, const u32x4& v) {
+        f32x4* d = reinterpret_cast<f32x4*>(to + 8 * idx);
+        d[0] = f32x4{lo2f(v.x), hi2f(v.x), lo2f(v.y), hi2f(v.y)};
+        d[1] = f32x4{lo2f(v.z), hi2f(v.z), lo2f(v.w), hi2f(v.w)};
+      };
+      widen(sk, kq4[r]);
+      widen(sq, qq4[r]);
+    }
+    sval[threadIdx.x] = bf2f(val);
+    if (threadIdx.x < kScanTokens) {
+      const float time_step = softplus(bf2f(al) + dth);
+      sgate[threadIdx.x] = float2{hexp(rbf(time_step * ah)), rbf(sigmoid(bf2f(be)))};
+    }
+  };
+  struct Token {
+    float k[KJ], q[KJ], value;
+    float2 gate;
+  };
+  auto read = [&](int tt, Token& v) {
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) {
+      v.k[j] = sk[tt * key_dim + lane + 32 * j];
+      v.q[j] = sq[tt * key_dim + lane + 32 * j];
+    }
+    v.value = sval[tt * CH + ch];
+    v.gate = sgate[tt];
+  };
+  float kept = 0.0f;
+  auto chain = [&](int tt, const Token& v) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) acc += s[j] * v.k[j];
+    const float total = sum32_everywhere(acc);
+    const float delta = (v.value - total * v.gate.x) * v.gate.y;
+    float acc2 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) {
+      s[j] = s[j] * v.gate.x + v.k[j] * delta;
+      acc2 += s[j] * v.q[j];
+    }
+    acc2 = sum32_everywhere(acc2);
+    kept = tt == lane ? acc2 : kept;
+  };
+  request(0);
   for (int t0 = 0; t0 < m; t0 += kScanTokens) {
     const int ts = min(kScanTokens, m - t0);
-    // stage: k and q rows lane-major, values, decay and rate
-    const int quads = key_dim >> 3;
-    for (int idx = threadIdx.x; idx < ts * quads; idx += blockDim.x) {
-      const int tt = idx / quads, qd = idx - tt * quads;
-      const size_t src = (size_t)(t0 + tt) * key_size + kbase + 8 * qd;
-      const u32x4 kq4 = *reinterpret_cast<const u32x4*>(k + src);
-      const u32x4 qq4 = *reinterpret_cast<const u32x4*>(q + src);
-      const uint32_t kw[4] = {kq4.x, kq4.y, kq4.z, kq4.w}, qw[4] = {qq4.x, qq4.y, qq4.z, qq4.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int i = 8 * qd + e;
-        const int dst = tt * key_dim + (i & 31) * kj + (i >> 5);
-        sk[dst] = (uint16_t)(kw[e >> 1] >> (16 * (e & 1)));
-        sq[dst] = (uint16_t)(qw[e >> 1] >> (16 * (e & 1)));
-      }
-    }
-    for (int idx = threadIdx.x; idx < ts * 8; idx += blockDim.x) {
-      const int tt = idx >> 3, cv = min(c0 + (idx & 7), value_size - 1);
-      sval[idx] = bf2f(conv[(size_t)(t0 + tt) * qkv_size + 2 * key_size + cv]);
-    }
-    if (threadIdx.x < ts) {
-      const int t = t0 + threadIdx.x;
-      const float time_step = softplus(bf2f(alpha[(size_t)t * value_heads + head]) + dth);
-      sdecay[threadIdx.x] = hexp(rbf(time_step * ah));
-      srate[threadIdx.x] = rbf(sigmoid(bf2f(beta[(size_t)t * value_heads + head])));
-    }
+    place();
+    if (t0 + kScanTokens < m) request(t0 + kScanTokens);
     __syncthreads();
-    for (int tt = 0; tt < ts; ++tt) {
-      const uint16_t* kr = sk + tt * key_dim + lane * kj;
-      const uint16_t* qr = sq + tt * key_dim + lane * kj;
-      float kv[KJ], qv[KJ];
-#pragma unroll
-      for (int j = 0; j < KJ; ++j) {
-        kv[j] = bf2f(kr[j]);
-        qv[j] = bf2f(qr[j]);
-      }
-      float acc = 0.0f;
-#pragma unroll
-      for (int j = 0; j < KJ; ++j) acc += s[j] * kv[j];
-      acc = tree32_lanes(acc);
-      const float t_lo = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 0));
-      const float t_hi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 32));
-      const float total = half ? t_hi : t_lo;
-      const float decay = sdecay[tt];
-      const float delta = (sval[tt * 8 + ch] - total * decay) * srate[tt];
-      float acc2 = 0.0f;
-#pragma unroll
-      for (int j = 0; j < KJ; ++j) {
-        s[j] = s[j] * decay + kv[j] * delta;
-        acc2 += s[j] * qv[j];
-      }
-      acc2 = tree32_lanes(acc2);
-      if (lane == 0 && valid) out[(size_t)(t0 + tt) * value_size + c] = f2bf(acc2 * scale);
+    Token x, y;
+    read(0, x);
+    int tt = 0;
+#pragma unroll 1
+    for (; tt + 2 <= ts; tt += 2) {
+      read(tt + 1, y);
+      chain(tt, x);
+      read(min(tt + 2, kScanTokens - 1), x);
+      chain(tt + 1, y);
     }
+    if (tt < ts) chain(tt, x);
+    sout[lane * CH + ch] = f2bf(kept * scale);
     __syncthreads();
+    if ((int)threadIdx.x < ts)
+      *reinterpret_cast<u32x4*>(out + (size_t)(t0 + threadIdx.x) * value_size + c0) =
+          reinterpret_cast<const u32x4*>(sout)[threadIdx.x];
   }
-  if (valid) {
 #pragma unroll
-    for (int j = 0; j < KJ; ++j) state[(size_t)c * key_dim + lane + 32 * j] = s[j];
-  }
+  for (int j = 0; j < KJ; ++j) state[(size_t)c * key_dim + lane + 32 * j] = s[j];
 }
 
 // RoPE tables [cos x R/2 | sin x R/2] for the chunk's positions

@@ -1693,10 +1693,13 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
           project(s->pf_x, H, W(4), VH, beta);
         }
         const int64_t conv_base = cap * d.KV_STRIDE + l * d.LIN;
-        L(KC_PREPARE_LINEAR, k_bprepare,
-          dim3((unsigned)((d.QKV + c.key_dim - 1) / c.key_dim), rows_n), dim3(kBlock), 0,
-          (const uint16_t*)qkv, (const uint16_t*)s->cache, conv_base, params, first,
-          (const float*)W(9), (int)d.QKV, c.key_dim, c.key_heads, conv, qn, kn);
+        // batched calls have key_dim 128
+        const bool few = rows_n <= 4 * kPrepareTokens;
+        const int prepare_tokens = few ? kPrepareFew : kPrepareTokens;
+        L(KC_PREPARE_LINEAR, few ? k_bprepare<128, kPrepareFew> : k_bprepare<128, kPrepareTokens>,
+          dim3((unsigned)((d.QKV + 127) / 128), (unsigned)((rows_n + prepare_tokens - 1) / prepare_tokens)), dim3(kBlock), 0,
+          (const uint16_t*)qkv, (const uint16_t*)s->cache, conv_base, params, first, rows_n,
+          (const float*)W(9), (int)d.QKV, c.key_heads, conv, qn, kn);
         L(KC_PREPARE_LINEAR, k_bhistory, dim3(grid_for((3 * d.QKV + kBlock - 1) / kBlock, 1024)),
           dim3(kBlock), 0, (const uint16_t*)qkv, rows_n, s->cache, conv_base, params, first,
           (int)d.QKV);
@@ -1705,12 +1708,14 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
         if (c.key_dim == 32) scan = k_bscan<1>;
         else if (c.key_dim == 64) scan = k_bscan<2>;
         else if (c.key_dim == 256) scan = k_bscan<8>;
-        L(KC_DELTA, scan, dim3((unsigned)((d.VS + 7) / 8)), dim3(kBlock), bscan_lds_bytes(c.key_dim),
+        L(KC_DELTA, scan, dim3((unsigned)(d.VS / 8)), dim3(kBlock), bscan_lds_bytes(c.key_dim),
           (const uint16_t*)conv, (const uint16_t*)qn, (const uint16_t*)kn, (const uint16_t*)alpha,
           (const uint16_t*)beta, (const float*)W(5), (const float*)W(6), s->shadow + l * d.REC,
-          rows_n, (int)d.VS, c.value_dim, VH, c.key_dim, c.key_heads, (int)d.QKV, scale, core);
-        L(KC_GATED_NORM, k_gated_norm, dim3((unsigned)(VH * rows_n)), dim3(kBlock), 0,
-          (const uint16_t*)core, (const uint16_t*)z, (const float*)W(7), c.value_dim, c.eps, gated);
+          rows_n, (int)d.VS, c.value_dim, VH, c.key_heads, (int)d.QKV, scale, core);
+        const int gated_rows = few ? 8 : kGatedRows;
+        L(KC_GATED_NORM, k_bgated_norm, dim3((unsigned)((VH * rows_n + gated_rows - 1) / gated_rows)), dim3(kBlock),
+          bgated_lds_bytes(c.value_dim), (const uint16_t*)core, (const uint16_t*)z, (const float*)W(7), VH * rows_n,
+          gated_rows, c.value_dim, c.eps, gated);
         residual_rows(gated, (int)d.VS, W(8), s->pf_h, s->pf_attn);
         post_norm = W(10);
         ffn = 11;
