@@ -780,6 +780,7 @@ struct cq35_session {
   float *pf_rope = nullptr, *pf_logits = nullptr, *pf_probs = nullptr, *pf_scratch = nullptr;
   float *pf_part = nullptr, *pf_spart = nullptr;  // matrix-core experts: routed / shared down sums
   int *pf_eoff = nullptr, *pf_order = nullptr;    // matrix-core experts: buckets
+  int* pf_tiles = nullptr;                        // matrix-core experts: tiles that hold work
   int* pf_ids = nullptr;
   uint32_t* pf_ranges = nullptr;  // k_bgemm: magnitude ranges of a launch's weight and token tiles
   int pf_attn_tokens = 0;  // tokens per staged-attention launch (scratch rows)
@@ -1510,6 +1511,7 @@ int setup_prefill(cq35_session* s) {
     check(dalloc(s, &s->pf_probs, m * d.K));
     check(dalloc(s, &s->pf_eoff, d.E + 2));
     check(dalloc(s, &s->pf_order, m * d.K));
+    check(dalloc(s, &s->pf_tiles, 1 + moe_tiles(m, d.K, d.E)));
     check(dalloc(s, &s->pf_part, m * d.K * d.H));
     check(dalloc(s, &s->pf_spart, m * d.H));
   }
@@ -1742,27 +1744,27 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
           c0 + rows_n == n ? s->ids + l * d.K : (int*)nullptr);
         const int rows = K * I + SI;
         if ((s->matrix & CQ35_MATRIX_EXPERTS) && H % 16 == 0 && I % 16 == 0 && SI % 16 == 0) {
-          const int A = rows_n * K;
-          L(KC_ROUTER, k_moe_bucket, dim3(1), dim3(1024), (size_t)E * 2 * sizeof(int),
-            (const int*)s->pf_ids, A, E, s->pf_eoff, s->pf_order);
-          const unsigned mt = (unsigned)((rows_n + 31) / 32);  // token tiles of the busiest expert at most
-          L(KC_MOE_GATE, k_mmoe_gate, dim3((unsigned)((std::max(I, SI) + kXRows - 1) / kXRows), (unsigned)(E + 1), mt),
+          L(KC_ROUTER, k_moe_bucket, dim3(1), dim3(1024), (size_t)E * 3 * sizeof(int),
+            (const int*)s->pf_ids, rows_n * K, E, s->pf_eoff, s->pf_order, rows_n, s->pf_tiles);
+          const int most = moe_tiles(rows_n, K, E);
+          const int gate_blocks = (std::max(I, SI) + kXRows - 1) / kXRows, down_blocks = (H + kXRows - 1) / kXRows;
+          L(KC_MOE_GATE, k_mmoe_gate, dim3(xtile_grid(gate_blocks, most)),
             dim3(64 * kXWaves), 0, (const uint16_t*)s->pf_x, H, (const uint16_t*)W(ffn + 1),
             (const uint16_t*)W(ffn + 2), (const uint16_t*)W(ffn + 5), (const uint16_t*)W(ffn + 6),
             (const int*)s->pf_eoff, (const int*)s->pf_order, (const float*)s->pf_probs,
-            (const float*)s->pf_logits, E, K, I, SI, rows_n, s->pf_act);
-          L(KC_MOE_DOWN, k_mmoe_down, dim3((unsigned)((H + kXRows - 1) / kXRows), (unsigned)(E + 1), mt),
+            (const float*)s->pf_logits, E, K, I, SI, rows_n, (const int*)s->pf_tiles, gate_blocks, s->pf_act);
+          L(KC_MOE_DOWN, k_mmoe_down, dim3(xtile_grid(down_blocks, most)),
             dim3(64 * kXWaves), 0, (const uint16_t*)s->pf_act, (const uint16_t*)W(ffn + 3),
             (const uint16_t*)W(ffn + 7), (const int*)s->pf_eoff, (const int*)s->pf_order, E, K, I, SI, H,
-            rows_n, s->pf_part, s->pf_spart);
+            rows_n, (const int*)s->pf_tiles, down_blocks, s->pf_part, s->pf_spart);
           L(KC_MOE_DOWN, k_moe_combine, dim3((unsigned)((H + kBlock - 1) / kBlock), (unsigned)rows_n),
             dim3(kBlock), 0, (const float*)s->pf_part, (const float*)s->pf_spart,
             (const uint16_t*)s->pf_attn, H, K, s->pf_h);
         } else {
           if (H <= 2048) {
             // the gate/up rows read once per chunk: assignments bucketed by expert
-            L(KC_ROUTER, k_moe_bucket, dim3(1), dim3(1024), (size_t)E * 2 * sizeof(int),
-              (const int*)s->pf_ids, rows_n * K, E, s->pf_eoff, s->pf_order);
+            L(KC_ROUTER, k_moe_bucket, dim3(1), dim3(1024), (size_t)E * 3 * sizeof(int),
+              (const int*)s->pf_ids, rows_n * K, E, s->pf_eoff, s->pf_order, rows_n, (int*)nullptr);
             auto grouped = [&](auto routed, auto shared) {
               L(KC_MOE_GATE, routed, dim3((unsigned)((I + kGRows - 1) / kGRows), (unsigned)E), dim3(kBlock), 0,
                 (const uint16_t*)s->pf_x, H, (const uint16_t*)W(ffn + 1), (const uint16_t*)W(ffn + 2),

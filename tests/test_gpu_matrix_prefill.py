@@ -191,3 +191,25 @@ def test_matrix_prefill_switch_leaves_decode_and_exact_path(oracle):
         la, ta = a.step_raw([ta])
         lb, tb = b.step_raw([tb])
         assert ta == tb and np.array_equal(la, lb)
+
+
+@pytest.mark.parametrize("name,n", [("mini-moe", 33), ("mini-moe", 290), ("mini-moe", 1061), ("tiny-moe", 35),
+                                    ("qwen36-35b-a3b@4", 65)])
+def test_expert_tiles_do_not_depend_on_the_call(name, n):
+    """The listed expert tiles (none, one or several per expert; one, four or
+    sixteen row blocks): each output is its own dot product, so one call and
+    two of other tile counts leave the same bits."""
+    cfg = shape(name)
+    say("expert tiles", name, n)
+    m = cq35.Model.synthetic(cfg, seed=23)
+    if cfg["key_dim"] != 128:
+        pytest.skip("multi-token calls run token by token")
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).tolist()
+    one, two = m.session(n + 3), m.session(n + 3)
+    for s in (one, two):
+        s.set_matrix_prefill(Session.MATRIX_EXPERTS)
+    logits, _ = one.step_raw(prompt)
+    two.step_raw(prompt[:n - n // 3])
+    again, _ = two.step_raw(prompt[n - n // 3:])
+    assert np.array_equal(logits, again)
+    assert np.array_equal(one.export_state(0), two.export_state(0))
