@@ -1487,7 +1487,15 @@ int setup_prefill(cq35_session* s) {
   if (s->pf_ready) return CQ35_OK;
   const Dims& d = s->model->d;
   const cq35_config& c = s->model->cfg;
-  const int64_t m = s->matrix ? kMChunk : kBChunk, VH = c.value_heads;
+  const int64_t VH = c.value_heads, limit = s->matrix ? kMChunk : kBChunk;
+  int64_t m = std::min(limit, (s->capacity + 15) / 16 * 16);
+  // a quarter of the rows where they would take an eighth of what is free
+  const int64_t row_bytes = 2 * (3 * d.H + std::max(d.QKV, 2 * d.QS) + std::max(d.VS, d.KVS) + std::max(2 * VH, d.KVS) +
+                                 std::max(d.QKV, d.QS) + 2 * d.KS + std::max(d.VS, d.QS) + d.VS +
+                                 std::max(d.I, d.K * d.I + d.SI)) + (c.moe ? 4 * ((d.K + 1) * d.H + d.E) : 0);
+  size_t free_bytes = 0, total_bytes = 0;
+  HIP_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
+  if (m * row_bytes > (int64_t)(free_bytes / 8)) m = std::min(m, limit / 4);
   s->pf_rows = (int)m;
   int rc = CQ35_OK;
   auto check = [&](int r) { if (r && !rc) rc = r; };

@@ -90,3 +90,11 @@ def test_batched_prefill_two_chunks_moe(oracle):
     cfg = cc.preset("mini-moe")
     prompt = np.random.default_rng(54).integers(0, cfg["vocab"], 300).tolist()
     run(oracle, "mini-moe", 17, [], prompt, 3)
+
+
+@pytest.mark.parametrize("name", ["mini", "mini-moe"])
+def test_batched_prefill_over_the_chunk_edge(oracle, name):
+    """1037 tokens: a full chunk of 1024 rows and a short one."""
+    cfg = cc.preset(name)
+    prompt = np.random.default_rng(55).integers(0, cfg["vocab"], 1037).tolist()
+    run(oracle, name, 18, [], prompt, 2)
