@@ -1444,13 +1444,13 @@ const char* prefill_unsupported(const cq35_model& m) {
 // whole call, at 5 / 8 tokens: 871 / 1073 us against 916 / 923 here).
 bool bgemm_ok(int n, int64_t cols) { return cols % 64 == 0 && n >= kBTokens; }
 
-template <int kMode, int TT, int RT>
-void bgemm_launch(Launcher& L, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2,
+template <int kMode, int TT, int RT, typename Launch>
+void bgemm_launch(Launch& L, int cus, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2,
                   const uint16_t* res, uint32_t* ranges) {
   using T = BGemmTile<TT, RT>;
   const int per = bgemm_rows<kMode, RT>();
   const int tr = (int)((seg_rows(seg) + per - 1) / per), tt = (n + T::kTokens - 1) / T::kTokens;
-  const int grid = std::min((tr + 7) / 8 * tt, std::max(L.s->model->cus / 8, 1) * T::kBlocksPerCu) * 8;
+  const int grid = std::min((tr + 7) / 8 * tt, std::max(cus / 8, 1) * T::kBlocksPerCu) * 8;
   L(KC_PREFILL_PROJECT, k_bgemm<kMode, TT, RT>, dim3((unsigned)grid), dim3(kEThreads), T::kLds, x, n, cols, seg, w2, res,
     ranges);
   L(KC_PREFILL_PROJECT, k_bgemm_fix<kMode, TT, RT>, dim3((unsigned)((tr * tt + kBlock - 1) / kBlock)), dim3(kBlock), 0, x,
@@ -1462,12 +1462,16 @@ void bgemm_launch(Launcher& L, const uint16_t* x, int n, int cols, const Segment
 // operands per product. 12352 rows x 2048 at 37 / 256 / 768 tokens: 59 / 240 /
 // 683 us against 69 / 262 / 653; the gate mode, with two row halves per tile,
 // turns earlier (6144 x 2048 twice at 16 / 128: 32 / 147 against 50 / 135).
-template <int kMode>
-void bgemm(Launcher& L, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2, const uint16_t* res,
-           uint32_t* ranges) {
-  if (n <= (kMode == kBGate ? 32 : 256)) bgemm_launch<kMode, 1, 1>(L, x, n, cols, seg, w2, res, ranges);
-  else bgemm_launch<kMode, 3, 1>(L, x, n, cols, seg, w2, res, ranges);
+template <int kMode, typename Launch>
+void bgemm(Launch& L, int cus, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2,
+           const uint16_t* res, uint32_t* ranges) {
+  if (n <= (kMode == kBGate ? 32 : 256)) bgemm_launch<kMode, 1, 1>(L, cus, x, n, cols, seg, w2, res, ranges);
+  else bgemm_launch<kMode, 3, 1>(L, cus, x, n, cols, seg, w2, res, ranges);
 }
+
+// Words of k_bgemm's ranges for launches of at most `rows` rows and n tokens:
+// kEWaves per tile of at least eight rows or sixteen tokens.
+int64_t bgemm_range_words(int64_t rows, int64_t n) { return rows + n + 2 * 8 * kEWaves; }
 
 hipError_t bgemm_lds_optin() {
   const std::pair<const void*, size_t> f[] = {
@@ -1511,7 +1515,7 @@ int setup_prefill(cq35_session* s) {
   check(dalloc(s, &s->pf_g, m * d.VS));                       // gated
   check(dalloc(s, &s->pf_act, m * std::max(d.I, d.K * d.I + d.SI)));
   check(dalloc(s, &s->pf_rope, m * std::max<int64_t>(d.R, 2)));
-  check(dalloc(s, &s->pf_ranges, std::max({d.QKV + d.VS + 2 * VH, 2 * d.QS + 2 * d.KVS, d.H, d.I}) + m + 2 * 8 * kEWaves));
+  check(dalloc(s, &s->pf_ranges, bgemm_range_words(std::max({d.QKV + d.VS + 2 * VH, 2 * d.QS + 2 * d.KVS, d.H, d.I}), m)));
   if (!rc && bgemm_lds_optin() != hipSuccess) rc = fail(CQ35_EDEVICE, "projection kernels' LDS");
   if (c.moe) {
     check(dalloc(s, &s->pf_logits, m * (d.E + 1)));
@@ -1576,7 +1580,7 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
         return true;
       }
       if (!mp && bgemm_ok(rows_n, cols)) {
-        bgemm<kBPlain>(L, x, rows_n, cols, seg, nullptr, nullptr, s->pf_ranges);
+        bgemm<kBPlain>(L, m.cus, x, rows_n, cols, seg, nullptr, nullptr, s->pf_ranges);
         return true;
       }
       return false;
@@ -1603,7 +1607,7 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
         L(KC_PREFILL_PROJECT, k_mproject<kBResidual>, mgrid(H, cols), dim3(64 * kMWaves), 0, x, rows_n, cols,
           (const uint16_t*)w, (const uint16_t*)nullptr, H, res, out);
       else if (!mp && bgemm_ok(rows_n, cols))
-        bgemm<kBResidual>(L, x, rows_n, cols, segments({{w, {out, H}}}), nullptr, res, s->pf_ranges);
+        bgemm<kBResidual>(L, m.cus, x, rows_n, cols, segments({{w, {out, H}}}), nullptr, res, s->pf_ranges);
       else
         L(KC_PREFILL_PROJECT, k_bproject<kBResidual>,
           dim3((unsigned)((H + bproject_rows<kBResidual>() - 1) / bproject_rows<kBResidual>()), tiles), dim3(kBlock), 0, x,
@@ -1819,7 +1823,7 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
               (const uint16_t*)s->pf_x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
               (int)d.I, (const uint16_t*)nullptr, s->pf_act);
         else if (!mp && bgemm_ok(rows_n, H))
-          bgemm<kBGate>(L, s->pf_x, rows_n, H, segments({{W(ffn), {s->pf_act, d.I}}}), (const uint16_t*)W(ffn + 1),
+          bgemm<kBGate>(L, m.cus, s->pf_x, rows_n, H, segments({{W(ffn), {s->pf_act, d.I}}}), (const uint16_t*)W(ffn + 1),
                         nullptr, s->pf_ranges);
         else
           L(KC_PREFILL_PROJECT, k_bproject<kBGate>, dim3((unsigned)d.I, tiles), dim3(kBlock), 0,
@@ -2975,6 +2979,68 @@ extern "C" int cq35_device_matrix_gemm(const uint16_t* x, const uint16_t* w, con
   for (uint16_t* p : {dx, dw, dw2, dres, dout})
     if (p) hipFree(p);
   if (e != hipSuccess) return fail(CQ35_EDEVICE, "device matrix GEMM: %s", hipGetErrorString(e));
+  return CQ35_OK;
+}
+
+namespace {
+
+// A Launcher for the default stream.
+struct DirectLauncher {
+  template <typename Kernel, typename... Args>
+  void operator()(int, Kernel kernel, dim3 grid, dim3 block, size_t lds, Args... args) {
+    kernel<<<grid, block, lds>>>(args...);
+  }
+};
+
+template <int kMode>
+void device_exact_gemm(int route, int cus, const uint16_t* x, int n, int cols, const uint16_t* w, const uint16_t* w2,
+                       int rows, const uint16_t* res, uint16_t* out, uint32_t* ranges) {
+  DirectLauncher L;
+  if (route == 1 && bgemm_ok(n, cols)) {
+    bgemm<kMode>(L, cus, x, n, cols, segments({{w, {out, rows}}}), w2, res, ranges);
+    return;
+  }
+  L(0, k_bproject<kMode>,
+    dim3((unsigned)((rows + bproject_rows<kMode>() - 1) / bproject_rows<kMode>()),
+         (unsigned)((n + 4 * kBTokens - 1) / (4 * kBTokens))),
+    dim3(kBlock), 0, x, n, cols, w, w2, rows, res, out);
+}
+
+}  // namespace
+
+extern "C" int cq35_device_exact_gemm(const uint16_t* x, const uint16_t* w, const uint16_t* w2, const uint16_t* res,
+                                      int64_t n, int64_t rows, int64_t cols, int mode, int kernel, uint16_t* out) {
+  if (!x || !w || !out || n <= 0 || rows <= 0 || cols <= 0 || cols % 8 || n > (1 << 20) || rows > (1 << 20) ||
+      cols > 65536 || mode < kBPlain || mode > kBGate || kernel < 0 || kernel > 1 || (mode == kBGate && !w2) ||
+      (mode == kBResidual && !res))
+    return fail(CQ35_EINVAL, "bad exact GEMM shape");
+  int device = 0, cus = 0;
+  uint16_t *dx = nullptr, *dw = nullptr, *dw2 = nullptr, *dres = nullptr, *dout = nullptr;
+  uint32_t* ranges = nullptr;
+  hipError_t e = hipGetDevice(&device);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+  if (e == hipSuccess) e = bgemm_lds_optin();
+  if (e == hipSuccess) e = hipMalloc(&dx, n * cols * 2);
+  if (e == hipSuccess) e = hipMalloc(&dw, rows * cols * 2);
+  if (e == hipSuccess && mode == kBGate) e = hipMalloc(&dw2, rows * cols * 2);
+  if (e == hipSuccess && mode == kBResidual) e = hipMalloc(&dres, n * rows * 2);
+  if (e == hipSuccess) e = hipMalloc(&dout, n * rows * 2);
+  if (e == hipSuccess) e = hipMalloc(&ranges, bgemm_range_words(rows, n) * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMemcpy(dx, x, n * cols * 2, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(dw, w, rows * cols * 2, hipMemcpyHostToDevice);
+  if (e == hipSuccess && dw2) e = hipMemcpy(dw2, w2, rows * cols * 2, hipMemcpyHostToDevice);
+  if (e == hipSuccess && dres) e = hipMemcpy(dres, res, n * rows * 2, hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    auto run = [&](auto f) { f(kernel, cus, dx, (int)n, (int)cols, dw, dw2, (int)rows, dres, dout, ranges); };
+    if (mode == kBPlain) run(device_exact_gemm<kBPlain>);
+    else if (mode == kBResidual) run(device_exact_gemm<kBResidual>);
+    else run(device_exact_gemm<kBGate>);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpy(out, dout, n * rows * 2, hipMemcpyDeviceToHost);
+  for (void* p : {(void*)dx, (void*)dw, (void*)dw2, (void*)dres, (void*)dout, (void*)ranges})
+    if (p) hipFree(p);
+  if (e != hipSuccess) return fail(CQ35_EDEVICE, "device exact GEMM: %s", hipGetErrorString(e));
   return CQ35_OK;
 }
 

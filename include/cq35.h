@@ -300,6 +300,15 @@ int cq35_device_gemv(const uint16_t* x, const uint16_t* w, int64_t rows, int64_t
 int cq35_device_matrix_gemm(const uint16_t* x, const uint16_t* w, const uint16_t* w2,
                             const uint16_t* res, int64_t n, int64_t rows, int64_t cols, int mode,
                             int kernel, uint16_t* out);
+/* Device exact product of the prompt projections (the reference's batched
+ * order, one accumulator per lane of 256) over host arrays laid out as above,
+ * cols a multiple of 8, the same epilogues. kernel 0: the vector kernel; 1:
+ * the kernels a prompt of n tokens runs (eight tokens or more of widths in
+ * whole 128-byte lines: the F32 matrix cores and the recomputation of what
+ * they would round differently). The same bits. */
+int cq35_device_exact_gemm(const uint16_t* x, const uint16_t* w, const uint16_t* w2,
+                           const uint16_t* res, int64_t n, int64_t rows, int64_t cols, int mode,
+                           int kernel, uint16_t* out);
 /* Device matrix-core attention of the prompt path (CQ35_MATRIX_ATTENTION's
  * kernel) over host arrays: n query rows at positions start .. start + n - 1
  * against keys 0 .. start + n - 1. q and gate [n][heads][head_dim] (q

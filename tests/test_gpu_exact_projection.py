@@ -2,16 +2,24 @@
 against the CPU restatement, bit for bit, where the kernel's tiling can go
 wrong: token counts around its 16- and 48-token tiles and the count at which
 it takes over, widths that leave a partial visit pair, a partial line group or
-a single visit, and row counts that end inside a tile. And the products that a
-fused multiply-add would round differently: value weights and inputs so small
-that the lowest bits of their products lie below the F32 subnormals,
-recomputed by k_bgemm_fix (with 300 tokens of 512 value channels some outputs
-differ where the fused sums are kept)."""
+a single visit, and row counts that end inside a tile.
+
+Then the products alone (cq35_device_exact_gemm), in every epilogue and both
+tile shapes, for the values that the route is chosen by: sums that show the
+order and the rounding of every step, products that are exact while their sums
+are subnormal (the matrix cores keep them), and what a fused multiply-add
+would round differently, recomputed by k_bgemm_fix: products whose lowest bits
+lie below the F32 subnormals, products beyond the largest F32, infinities and
+NaN. Against the batched order in numpy F32, which is the restatement's (first
+test); where the fix matters, the fused sums are shown to differ first."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import cq35
 import cq35.config as cc
+from cq35 import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +75,181 @@ def test_products_below_the_exact_range(oracle, tokens):
     print("exact projection, tiny weights", tokens, flush=True)
     prompt = np.random.default_rng(tokens).integers(0, cfg["vocab"], tokens).tolist()
     compare(oracle, cfg, weights, prompt)
+
+
+# ------------------------------------------------------- the products alone
+
+
+def widen(bits):
+    return (np.asarray(bits, np.uint16).astype(np.uint32) << 16).view(np.float32)
+
+
+def narrow(f):  # nearest even, NaN quieted
+    u = np.ascontiguousarray(f, np.float32).view(np.uint32).astype(np.uint64)
+    r = ((u + 0x7fff + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    return np.where(np.isnan(f), ((u >> 16) | 0x40).astype(np.uint16), r)
+
+
+def b256(x, w, fused=False):
+    """F32 totals [n][rows] of the batched order: lane l of 256 adds the low
+    and the high product of its pairs l, l + 256, ... to one accumulator, then
+    the lanes' halving tree. `fused`: each product and its sum rounded once
+    (through F64: off at most where F64 rounds the sum itself)."""
+    (n, cols), rows = x.shape, w.shape[0]
+    visits = -(-cols // 512)
+    pad = lambda a: np.pad(widen(a), ((0, 0), (0, 512 * visits - cols))).reshape(len(a), visits, 256, 2)
+    xs, ws = pad(x), pad(w)
+    acc = np.zeros((n, rows, 256), np.float32)
+    with np.errstate(all="ignore"):
+        for v in range(visits):
+            for half in range(2):
+                a, b = xs[:, None, v, :, half], ws[None, :, v, :, half]
+                if fused:
+                    acc = (acc.astype(np.float64) + a.astype(np.float64) * b.astype(np.float64)).astype(np.float32)
+                else:
+                    acc = acc + a * b
+        while acc.shape[-1] > 1:
+            h = acc.shape[-1] // 2
+            acc = acc[..., :h] + acc[..., h:]
+    return acc[..., 0]
+
+
+def silu(x):
+    x = np.ascontiguousarray(x, np.float32)
+    y = np.empty_like(x)
+    fp = ctypes.POINTER(ctypes.c_float)
+    assert _lib.load().cq35_device_numeric(1, x.ctypes.data_as(fp), y.ctypes.data_as(fp), x.size) == 0
+    return y
+
+
+def epilogue(mode, total, up, res):
+    with np.errstate(all="ignore"):
+        if mode == 0:
+            return narrow(total)
+        if mode == 1:
+            return narrow(widen(narrow(total)) + widen(res))
+        return narrow(widen(narrow(silu(widen(narrow(total))))) * widen(narrow(up)))
+
+
+def exact_gemm(x, w, w2, res, mode, kernel):
+    (n, cols), rows = x.shape, w.shape[0]
+    out = np.empty((n, rows), np.uint16)
+    ptr = lambda a: a.ctypes.data if a is not None else None
+    rc = _lib.load().cq35_device_exact_gemm(ptr(x), ptr(w), ptr(w2), ptr(res), n, rows, cols, mode, kernel, ptr(out))
+    assert rc == 0, _lib.load().cq35_last_error()
+    return out
+
+
+def odd(rng, shape, exponent):
+    """+-(an odd whole number of eight bits) * 2^exponent."""
+    m = rng.integers(64, 128, shape) * 2 + 1
+    return narrow((np.where(rng.random(shape) < 0.5, -m, m) * 2.0 ** exponent).astype(np.float32))
+
+
+def operands(kind, mode, n, rows, cols, rng):
+    """x, w, w2, res and whether the fused sums have to differ."""
+    x = narrow(rng.standard_normal((n, cols)).astype(np.float32))
+    w = narrow((rng.standard_normal((rows, cols)) * 0.05).astype(np.float32))
+    w2 = narrow((rng.standard_normal((rows, cols)) * 0.05).astype(np.float32)) if mode == 2 else None
+    res = narrow(rng.standard_normal((n, rows)).astype(np.float32)) if mode == 1 else None
+    differs = False
+    if kind == "cancelling":
+        # four lanes: products of +-2^18 that cancel within the lane, small
+        # ones between them whose low bits go where the order says
+        w[:] = 0
+        for lane in (0, 5, 130, 255):
+            c = np.array([512 * v + 2 * lane + h for v in range(-(-cols // 512)) for h in (0, 1)])
+            c = c[c < cols]
+            big = rng.permutation(len(c))[:len(c) // 4 * 2]
+            big.sort()
+            x[:, c] = narrow(rng.uniform(1, 2, (n, len(c))).astype(np.float32))
+            w[:, c] = narrow(rng.uniform(-2, 2, (rows, len(c))).astype(np.float32))
+            x[:, c[big]] = narrow(np.float32([512.0]))
+            w[:, c[big]] = narrow(np.where(np.arange(len(big)) % 2, -512.0, 512.0).astype(np.float32))
+    elif kind == "subnormal sums":
+        # products odd * 2^-149: exact, their sums below 2^-126
+        x, w = odd(rng, (n, cols), -70), odd(rng, (rows, cols), -79)
+        w = np.where(rng.random((rows, cols)) < 0.25, w, 0).astype(np.uint16)
+        if mode == 1:
+            res = narrow((rng.integers(-64, 64, (n, rows)) * 2.0 ** -132).astype(np.float32))
+        if mode == 2:
+            w2 = narrow(rng.standard_normal((rows, cols)).astype(np.float32) * np.float32(2.0 ** 60))
+    elif kind == "tiny":
+        # in one row tile, in turn an odd multiple of 2^-149 and an odd one of
+        # 2^-150: the halves are ties, to even before the sum or with it. The
+        # second's residues of 4 make the sums apart by a unit a pair; signs
+        # keep them below 2^-126, where BF16 has 2^16 units.
+        tile = 8 if mode == 2 else 16
+        m = rng.integers(32, 64, (n, cols)) * 4 + 1
+        x = narrow((m * np.where(np.arange(cols) % 2, 2.0 ** -71, 2.0 ** -70)).astype(np.float32))
+        m = rng.integers(32, 64, (tile, cols)) * 4
+        small = narrow((np.where(rng.random(m.shape) < 0.5, m + 1, -(m + 3)) * 2.0 ** -79).astype(np.float32))
+        w = narrow(rng.standard_normal((rows, cols)).astype(np.float32) * np.float32(2.0 ** 60))
+        if mode == 2:  # ordinary gates over such up sums, and the other way round
+            w2 = w.copy()
+            w2[tile:2 * tile] = small
+            w[2 * tile:3 * tile] = small
+        else:
+            w[tile:2 * tile] = small
+        if mode == 1:
+            res = narrow((rng.integers(-64, 64, (n, rows)) * 2.0 ** -132).astype(np.float32))
+        differs = True
+    elif kind == "huge":
+        # -1.5 * 2^127 + 2^128 in one lane: beyond the largest F32 in between
+        for t in (1, n - 1):
+            x[t, 10:12] = narrow(np.float32([2.0 ** 64, 2.0 ** 64]))
+        beyond = narrow(np.float32([-1.5 * 2.0 ** 63, 2.0 ** 64]))
+        w[:, 10:12] = 0
+        w[rows - 1, 10:12] = beyond
+        if mode == 2:
+            w2[:, 10:12] = 0
+            w2[0, 10:12] = beyond
+        differs = True
+    elif kind == "not finite":
+        x[n // 2, 3] = narrow(np.float32([np.inf]))[0]
+        x[n - 1, 4] = narrow(np.float32([np.nan]))[0]
+        w[1, 7] = narrow(np.float32([-np.inf]))[0]
+        w[rows - 1, 0] = narrow(np.float32([np.nan]))[0]
+        if mode == 2:
+            w2[2, 9] = narrow(np.float32([np.inf]))[0]
+    elif kind == "zeros":
+        x[:], w[:2 * 16] = 0x8000, 0
+    return x, w, w2, res, differs
+
+
+# 17 tokens: 16 x 16 tiles in every mode; 49 tokens: 48 x 16 in gate mode; 300
+# tokens: 48 x 16 in all. 36 rows (plain, residual: three row tiles, gate:
+# five) end inside a tile.
+@pytest.mark.parametrize("mode, n", [(0, 17), (0, 300), (1, 17), (1, 300), (2, 17), (2, 49)])
+@pytest.mark.parametrize("kind", ["ordinary", "cancelling", "subnormal sums", "tiny", "huge", "not finite", "zeros"])
+def test_products_alone(kind, mode, n):
+    rows, cols = 36, {"tiny": 4096, "cancelling": 2112}.get(kind, 1088)
+    print("exact products", kind, "mode", mode, "tokens", n, flush=True)
+    rng = np.random.default_rng(100 * mode + n)
+    x, w, w2, res, differs = operands(kind, mode, n, rows, cols, rng)
+    up = b256(x, w2) if mode == 2 else None
+    want = epilogue(mode, b256(x, w), up, res)
+    nan = np.isnan(widen(want))
+    if differs:
+        fused = epilogue(mode, b256(x, w, True), b256(x, w2, True) if mode == 2 else None, res)
+        assert ((fused != want) & ~(nan & np.isnan(widen(fused)))).sum() >= 2, "the values do not tell the routes apart"
+    if kind == "cancelling":
+        assert (b256(x[:, ::-1], w[:, ::-1]) != b256(x, w)).mean() > 0.9, "the order does not show"
+    if kind == "subnormal sums":
+        total = np.abs(b256(x, w))
+        assert (total < 2.0 ** -126).mean() > 0.5 and (widen(narrow(total)) > 0).mean() > 0.8
+    for kernel in (0, 1):
+        got = exact_gemm(x, w, w2, res, mode, kernel)
+        assert np.array_equal(nan, np.isnan(widen(got))), (kernel, "NaN")
+        assert np.array_equal(got[~nan], want[~nan]), (kernel, int((got[~nan] != want[~nan]).sum()))
+
+
+def test_numpy_order_is_the_restatement(oracle):
+    rng = np.random.default_rng(9)
+    for kind in ("ordinary", "cancelling", "subnormal sums", "tiny", "huge"):
+        x, w, _, _, _ = operands(kind, 0, 3, 32, 2112, rng)
+        total = b256(x, w)
+        for t in range(3):
+            for r in range(32):
+                assert np.float32(oracle.dot_b256(x[t], w[r])).view(np.uint32) == total[t, r].view(np.uint32) or \
+                    np.isnan(total[t, r])
