@@ -113,13 +113,6 @@ __device__ __forceinline__ uint32_t range_of(const uint32_t* ranges, int tile) {
 template <int kMode, int RT>
 constexpr int bgemm_rows() { return kMode == kBGate ? 8 * RT : 16 * RT; }
 
-template <int kMode>
-__device__ __forceinline__ uint16_t b_epilogue(float v, float v2, const uint16_t* res, size_t o) {
-  if (kMode == kBPlain) return f2bf(v);
-  if (kMode == kBResidual) return bf_add(f2bf(v), res[o]);
-  return bf_mul(f2bf(silu(rbf(v))), f2bf(v2));
-}
-
 // out_s[t][r] of n token rows against the concatenated rows of `seg` (gate
 // mode: one segment, w2 the up matrix), k_bproject's epilogues. cols % 64 ==
 // 0. One block per CU walks its tiles, the next tile's first stage requested
@@ -406,43 +399,63 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
   }
 }
 
-// The tiles of a k_bgemm launch whose products may not be exact, recomputed
-// in the separate-rounding order, one wave per output (k_bproject's order).
+// What a k_bgemm launch may have rounded differently, in the
+// separate-rounding order (b256_rows): groups of four waves look at
+// k_bproject's regions (bproject_rows rows, kBTokens tokens per wave), 64 at a
+// time, and run those that lie in such a pair of tiles. Row group g of token
+// group t is group (g + 8 t) mod `groups`'s, so that the regions of one weight
+// tile, of one token and of a whole matrix all spread over the chip while the
+// groups at work share a token group. With nothing to do 4.6 us, a launch's
+// own; everything, 12352 rows x 2048 columns x 777 tokens, 1.71 ms (11.5 T
+// multiply-adds/s, k_bproject's rate). Four 2B layers of a 777-token prompt:
+// 9.1 ms, 9.8 with one inexact row tile in every matrix, 32 with nothing
+// exact (one block per 256 tiles, recomputing alone: 118 and 1510).
+constexpr int kFixThreads = 1024, kFixGroups = kFixThreads / 256;
+
 template <int kMode, int TT, int RT>
-__global__ __launch_bounds__(kBlock) void k_bgemm_fix(const uint16_t* __restrict__ x, int n, int cols, Segments seg,
-                                                      const uint16_t* __restrict__ w2,
-                                                      const uint16_t* __restrict__ res,
-                                                      const uint32_t* __restrict__ ranges) {
+__global__ __launch_bounds__(kFixThreads) void k_bgemm_fix(const uint16_t* __restrict__ x, int n, int cols, Segments seg,
+                                                           const uint16_t* __restrict__ w2,
+                                                           const uint16_t* __restrict__ res,
+                                                           const uint32_t* __restrict__ ranges) {
   using T = BGemmTile<TT, RT>;
-  constexpr int kBlockRows = bgemm_rows<kMode, RT>();
+  constexpr int kBlockRows = bgemm_rows<kMode, RT>(), R = bproject_rows<kMode>();
+  static_assert(kBlockRows % R == 0 && T::kTokens % kBTokens == 0, "a region lies in one tile");
   const int rows = seg.rows[0] + seg.rows[1] + seg.rows[2] + seg.rows[3];
   const int tiles_t = (n + T::kTokens - 1) / T::kTokens, tiles_r = (rows + kBlockRows - 1) / kBlockRows;
-  const int tiles = tiles_t * tiles_r;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int base = blockIdx.x * kBlock; base < tiles; base += gridDim.x * kBlock) {
-    // each wave looks at all of the block's tiles, 64 at a time
-    for (int k = 0; k < kBlock && base + k < tiles; k += 64) {
-      const int mine = base + k + lane;
-      const bool bad = mine < tiles && !bf_products_exact(range_of(ranges, tiles_r + mine % tiles_t), range_of(ranges, mine / tiles_t));
-      for (unsigned long long todo = __ballot(bad); todo; todo &= todo - 1) {
-        const int tile = base + k + __ffsll(todo) - 1, tile_t = tile % tiles_t, tile_r = tile / tiles_t;
-        for (int i = wave; i < T::kTokens * kBlockRows; i += kBlock / 64) {
-          const int t = tile_t * T::kTokens + i / kBlockRows, r = tile_r * kBlockRows + i % kBlockRows;
-          if (t >= n || r >= rows) continue;  // uniform per wave
-          int local;
-          const int s = segment_of(seg, r, &local);
-          const int srows = s == 0 ? seg.rows[0] : s == 1 ? seg.rows[1] : s == 2 ? seg.rows[2] : seg.rows[3];
-          float a[4] = {0.0f, 0.0f, 0.0f, 0.0f}, a2[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-          for (int q = lane; q < (cols >> 3); q += 64) {
-            const u32x4 xq = ldq(x + (size_t)t * cols, q);
-            b256_acc(a, xq, ldq(segment_w(seg, s) + (size_t)local * cols, q));
-            if (kMode == kBGate) b256_acc(a2, xq, ldq(w2 + (size_t)local * cols, q));
-          }
-          const float v = b256_tree(a), v2 = kMode == kBGate ? b256_tree(a2) : 0.0f;
-          const size_t at = (size_t)t * srows + local;
-          if (lane == 0) segment_out(seg, s)[at] = b_epilogue<kMode>(v, v2, res, at);
-        }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int groups = (int)gridDim.x * kFixGroups, group = (int)blockIdx.x + (int)gridDim.x * (wave >> 2);
+  const int groups_r = (rows + R - 1) / R, groups_t = (n + 4 * kBTokens - 1) / (4 * kBTokens);
+  const int each = (groups_r + groups - 1) / groups;  // row groups per token group, at most
+  for (int base = 0; base < each * groups_t; base += 64) {
+    auto place = [&](int i, int* row0, int* t0) {  // the group's region i, if there is one
+      const int t = i / each, turn = (group - 8 * t) % groups;
+      const int g = (turn < 0 ? turn + groups : turn) + i % each * groups;
+      *row0 = g * R;
+      *t0 = (t * 4 + (wave & 3)) * kBTokens;
+      return t < groups_t && g < groups_r && *t0 < n;
+    };
+    int row0, t0;
+    const bool bad = place(base + lane, &row0, &t0) &&
+                     !bf_products_exact(range_of(ranges, tiles_r + t0 / T::kTokens), range_of(ranges, row0 / kBlockRows));
+    for (unsigned long long todo = __ballot(bad); todo; todo &= todo - 1) {
+      place(base + __ffsll(todo) - 1, &row0, &t0);
+      const uint16_t* w[R];
+      const uint16_t* up = nullptr;
+      uint16_t* out[R];
+      int local[R], srows[R];
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const int s = segment_of(seg, min(row0 + k, rows - 1), &local[k]);
+        w[k] = segment_w(seg, s) + (size_t)local[k] * cols;
+        if (kMode == kBGate) up = w2 + (size_t)local[k] * cols;
+        out[k] = segment_out(seg, s);
+        srows[k] = s == 0 ? seg.rows[0] : s == 1 ? seg.rows[1] : s == 2 ? seg.rows[2] : seg.rows[3];
       }
+      b256_rows<kMode>(x, n, cols, w, up, t0, [&](int k, int t, float v, float v2) {
+        if (row0 + k >= rows) return;
+        const size_t o = (size_t)t * srows[k] + local[k];
+        out[k][o] = b_epilogue<kMode>(v, v2, res, o);
+      });
     }
   }
 }

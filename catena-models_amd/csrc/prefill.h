@@ -66,22 +66,20 @@ enum { kBPlain = 0, kBResidual = 1, kBGate = 2 };
 template <int kMode>
 constexpr int bproject_rows() { return kMode == kBGate ? 1 : 2; }
 
-template <int kMode>
-__global__ __launch_bounds__(kBlock) void k_bproject(const uint16_t* __restrict__ x, int n,
-                                                     int cols, const uint16_t* __restrict__ w,
-                                                     const uint16_t* __restrict__ w2, int rows,
-                                                     const uint16_t* __restrict__ res,
-                                                     uint16_t* __restrict__ out) {
+// One wave's B256 sums of R rows (gate mode: a gate row of w and an up row of
+// w2) over the tokens t0 .. t0 + kBTokens - 1 below n: emit(row k, token,
+// total, up total) on lane 0.
+template <int kMode, typename Emit>
+__device__ __forceinline__ void b256_rows(const uint16_t* __restrict__ x, int n, int cols,
+                                          const uint16_t* const (&w)[bproject_rows<kMode>()], const uint16_t* w2, int t0,
+                                          Emit emit) {
   constexpr int R = bproject_rows<kMode>();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row0 = blockIdx.x * R;
-  const int t0 = (blockIdx.y * 4 + wave) * kBTokens;
-  if (t0 >= n || row0 >= rows) return;  // wave-uniform
+  const int lane = threadIdx.x & 63;
   const int quads = cols >> 3;
   const u32x4* wr[R];
 #pragma unroll
-  for (int k = 0; k < R; ++k) wr[k] = reinterpret_cast<const u32x4*>(w + (size_t)min(row0 + k, rows - 1) * cols);
-  const u32x4* wr2 = kMode == kBGate ? reinterpret_cast<const u32x4*>(w2 + (size_t)row0 * cols) : nullptr;
+  for (int k = 0; k < R; ++k) wr[k] = reinterpret_cast<const u32x4*>(w[k]);
+  const u32x4* wr2 = reinterpret_cast<const u32x4*>(w2);
   float acc[R][kBTokens][4], acc2[kMode == kBGate ? kBTokens : 1][4];
 #pragma unroll
   for (int t = 0; t < kBTokens; ++t)
@@ -127,24 +125,42 @@ __global__ __launch_bounds__(kBlock) void k_bproject(const uint16_t* __restrict_
     }
   }
 #pragma unroll
-  for (int k = 0; k < R; ++k) {
-    const int row = row0 + k;
-    if (row >= rows) break;  // wave-uniform
+  for (int k = 0; k < R; ++k)
 #pragma unroll
     for (int t = 0; t < kBTokens; ++t) {
       if (t0 + t >= n) break;  // wave-uniform
-      const float total = tot[k][t];
-      const float total2 = kMode == kBGate ? tot2[t] : 0.0f;
-      if (lane == 0) {
-        const size_t o = (size_t)(t0 + t) * rows + row;
-        uint16_t y;
-        if (kMode == kBPlain) y = f2bf(total);
-        else if (kMode == kBResidual) y = bf_add(f2bf(total), res[o]);
-        else y = bf_mul(f2bf(silu(rbf(total))), f2bf(total2));
-        out[o] = y;
-      }
+      if (lane == 0) emit(k, t0 + t, tot[k][t], kMode == kBGate ? tot2[t] : 0.0f);
     }
-  }
+}
+
+// The epilogues over the totals of output element o.
+template <int kMode>
+__device__ __forceinline__ uint16_t b_epilogue(float v, float v2, const uint16_t* res, size_t o) {
+  if (kMode == kBPlain) return f2bf(v);
+  if (kMode == kBResidual) return bf_add(f2bf(v), res[o]);
+  return bf_mul(f2bf(silu(rbf(v))), f2bf(v2));
+}
+
+template <int kMode>
+__global__ __launch_bounds__(kBlock) void k_bproject(const uint16_t* __restrict__ x, int n,
+                                                     int cols, const uint16_t* __restrict__ w,
+                                                     const uint16_t* __restrict__ w2, int rows,
+                                                     const uint16_t* __restrict__ res,
+                                                     uint16_t* __restrict__ out) {
+  constexpr int R = bproject_rows<kMode>();
+  const int wave = threadIdx.x >> 6;
+  const int row0 = blockIdx.x * R;
+  const int t0 = (blockIdx.y * 4 + wave) * kBTokens;
+  if (t0 >= n || row0 >= rows) return;  // wave-uniform
+  const uint16_t* wr[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) wr[k] = w + (size_t)min(row0 + k, rows - 1) * cols;
+  b256_rows<kMode>(x, n, cols, wr, kMode == kBGate ? w2 + (size_t)row0 * cols : nullptr, t0,
+                   [&](int k, int t, float total, float total2) {
+                     if (row0 + k >= rows) return;
+                     const size_t o = (size_t)t * rows + row0 + k;
+                     out[o] = b_epilogue<kMode>(total, total2, res, o);
+                   });
 }
 
 // Embedding rows of tokens [first, first + m) of the call (prefill.embed,

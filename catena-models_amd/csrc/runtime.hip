@@ -1453,8 +1453,8 @@ void bgemm_launch(Launch& L, int cus, const uint16_t* x, int n, int cols, const 
   const int grid = std::min((tr + 7) / 8 * tt, std::max(cus / 8, 1) * T::kBlocksPerCu) * 8;
   L(KC_PREFILL_PROJECT, k_bgemm<kMode, TT, RT>, dim3((unsigned)grid), dim3(kEThreads), T::kLds, x, n, cols, seg, w2, res,
     ranges);
-  L(KC_PREFILL_PROJECT, k_bgemm_fix<kMode, TT, RT>, dim3((unsigned)((tr * tt + kBlock - 1) / kBlock)), dim3(kBlock), 0, x,
-    n, cols, seg, w2, res, (const uint32_t*)ranges);
+  L(KC_PREFILL_PROJECT, k_bgemm_fix<kMode, TT, RT>, dim3((unsigned)cus), dim3(kFixThreads), 0, x, n, cols, seg, w2,
+    res, (const uint32_t*)ranges);
 }
 
 // Few tokens: 16 x 16 tiles, two blocks per CU (more tiles to spread and one
@@ -3010,7 +3010,7 @@ void device_exact_gemm(int route, int cus, const uint16_t* x, int n, int cols, c
 
 extern "C" int cq35_device_exact_gemm(const uint16_t* x, const uint16_t* w, const uint16_t* w2, const uint16_t* res,
                                       int64_t n, int64_t rows, int64_t cols, int mode, int kernel, uint16_t* out) {
-  if (!x || !w || !out || n <= 0 || rows <= 0 || cols <= 0 || cols % 8 || n > (1 << 20) || rows > (1 << 20) ||
+  if (!x || !w || !out || n <= 0 || rows <= 0 || cols <= 0 || cols % 8 || n > (1 << 16) || rows > (1 << 16) ||
       cols > 65536 || mode < kBPlain || mode > kBGate || kernel < 0 || kernel > 1 || (mode == kBGate && !w2) ||
       (mode == kBResidual && !res))
     return fail(CQ35_EINVAL, "bad exact GEMM shape");
