@@ -27,8 +27,11 @@ constexpr int kBTokens = 8;   // tokens per wave sharing each weight quad
 // exact 35B, 512 tokens 21.7 ms at 256 rows, 19.5 here; exact 2B, 777 tokens
 // 19.5 and 17.0; matrix 35B, 4000 tokens 32.3 ms at 1024 rows, 26.8 here. A
 // 35B row takes 0.16 MB.
-constexpr int kBChunk = 1024;
-constexpr int kMChunk = 2048;
+constexpr int64_t kBChunk = 1024;
+constexpr int64_t kMChunk = 2048;
+// Where memory is short.
+constexpr int64_t kBFewRows = 256;
+constexpr int64_t kMFewRows = 1024;
 
 __device__ __forceinline__ void b256_acc(float (&a)[4], const u32x4& x, const u32x4& w) {
   a[0] = (a[0] + lo2f(x.x) * lo2f(w.x)) + hi2f(x.x) * hi2f(w.x);

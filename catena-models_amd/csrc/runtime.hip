@@ -27,6 +27,7 @@
 #include "bgemm.h"
 #include "mfma.h"
 #include "gguf.h"
+#include "workspace.h"
 #include "batch.h"
 #include "batch_moe.h"
 
@@ -53,6 +54,38 @@ static int fail(int code, const char* fmt, ...) {
       return fail(CQ35_EDEVICE, "%s failed: %s (%s:%d)", #expr, hipGetErrorString(e_),     \
                   __FILE__, __LINE__);                                                    \
   } while (0)
+
+namespace {
+
+struct HipMemory {
+  static void* allocate(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    hipGetLastError();  // not the next launch's
+    return nullptr;
+  }
+  static void release(void* p) { hipFree(p); }
+};
+
+// The chunk buffers lent to the multi-token calls of a device's models.
+BlockPool<HipMemory>& device_pool(int device) {
+  static BlockPool<HipMemory> pools[64];
+  return pools[device & 63];
+}
+
+// hipMalloc on the current device; its idle chunk buffers make way.
+template <typename T>
+hipError_t device_malloc(T** p, size_t bytes) {
+  hipError_t e = hipMalloc((void**)p, bytes);
+  int device = 0;
+  if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && device_pool(device).trim()) {
+    hipGetLastError();
+    e = hipMalloc((void**)p, bytes);
+  }
+  return e;
+}
+
+}  // namespace
 
 extern "C" const char* cq35_last_error(void) { return g_error.c_str(); }
 extern "C" int cq35_abi_version(void) { return CQ35_ABI_VERSION; }
@@ -357,8 +390,11 @@ struct cq35_model {
   std::vector<void*> owned;   // allocations to free
   float* freq = nullptr;      // F32 theta^(-2i/R) (src/catena.rs:185-232)
   int64_t weight_bytes = 0;
+  std::once_flag prefill_once;  // prefill_kernels
+  hipError_t prefill_ready = hipSuccess;
   std::mutex batch_lock;      // one weight-shared batched step at a time
   BatchWorkspace* batch = nullptr;  // its buffers (allocated on first use)
+  bool pooled = false;              // counted by device_pool
 };
 
 namespace {
@@ -369,8 +405,10 @@ int finish_model(cq35_model* m) {
   std::vector<float> f(std::max(half, 1));
   for (int i = 0; i < half; ++i)
     f[i] = powf(m->cfg.theta, -((float)(2 * i) / (float)m->cfg.rope_dim));
-  HIP_TRY(hipMalloc(&m->freq, f.size() * sizeof(float)));
+  HIP_TRY(device_malloc(&m->freq, f.size() * sizeof(float)));
   HIP_TRY(hipMemcpy(m->freq, f.data(), f.size() * sizeof(float), hipMemcpyHostToDevice));
+  device_pool(m->device).enter();
+  m->pooled = true;
   return CQ35_OK;
 }
 
@@ -384,6 +422,7 @@ extern "C" int cq35_model_free(cq35_model* m) {
   destroy_batch(m->batch);
   for (void* p : m->owned) hipFree(p);
   if (m->freq) hipFree(m->freq);
+  if (m->pooled) device_pool(m->device).leave();
   delete m;
   return CQ35_OK;
 }
@@ -410,7 +449,7 @@ extern "C" int cq35_model_create(const cq35_config* cfg, const void* const* weig
     } else {
       if (i == n - 1 && weights[i] == weights[0]) { m->w[i] = m->w[0]; continue; }  // tied head
       void* p = nullptr;
-      hipError_t e = hipMalloc(&p, bytes);
+      hipError_t e = device_malloc(&p, bytes);
       if (e == hipSuccess) e = hipMemcpy(p, weights[i], bytes, hipMemcpyHostToDevice);
       if (e != hipSuccess) {
         if (p) hipFree(p);
@@ -650,7 +689,7 @@ extern "C" int cq35_model_create_synthetic(const cq35_config* cfg, uint64_t seed
     if (cfg->tied && i == n - 1) { m->w[i] = m->w[0]; continue; }  // lm_head = token_embd
     const int64_t bytes = tensor_bytes(t);
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = device_malloc(&p, bytes);
     if (e != hipSuccess) {
       cq35_model_free(m);
       return fail(CQ35_EDEVICE, "allocating weight %lld (%lld bytes): %s", (long long)i,
@@ -771,20 +810,7 @@ struct cq35_session {
   const void* mega_kernel = nullptr;  // k_decode_step<shape> for this model
   int mega_lds = 0;                   // its dynamic LDS bytes
   uint32_t seq = 0;
-  // batched prefill: chunk buffers of kBChunk token rows, allocated on the
-  // first multi-token call at key_dim 128
-  bool pf_ready = false;
-  uint16_t *pf_h = nullptr, *pf_x = nullptr, *pf_attn = nullptr;
-  uint16_t *pf_a = nullptr, *pf_b = nullptr, *pf_c = nullptr, *pf_d = nullptr;
-  uint16_t *pf_e = nullptr, *pf_f = nullptr, *pf_g = nullptr, *pf_act = nullptr;
-  float *pf_rope = nullptr, *pf_logits = nullptr, *pf_probs = nullptr, *pf_scratch = nullptr;
-  float *pf_part = nullptr, *pf_spart = nullptr;  // matrix-core experts: routed / shared down sums
-  int *pf_eoff = nullptr, *pf_order = nullptr;    // matrix-core experts: buckets
-  int* pf_tiles = nullptr;                        // matrix-core experts: tiles that hold work
-  int* pf_ids = nullptr;
-  uint32_t* pf_ranges = nullptr;  // k_bgemm: magnitude ranges of a launch's weight and token tiles
-  int pf_attn_tokens = 0;  // tokens per staged-attention launch (scratch rows)
-  int pf_rows = 0;         // token rows of the chunk buffers
+  int prefill_rows = 0;    // token rows per chunk of multi-token calls (0: the rule of prefill_buffers)
   int matrix = 0;          // CQ35_MATRIX_* components of multi-token calls on MFMA
   int matrix_decode = 0;   // weight-shared batched decode products on MFMA
   int64_t split_keys = CQ35_SPLIT_KEYS_DEFAULT;  // decode attention splits above this many keys
@@ -801,7 +827,7 @@ namespace {
 template <typename T>
 int dalloc(cq35_session* s, T** p, int64_t count) {
   void* q = nullptr;
-  HIP_TRY(hipMalloc(&q, std::max<int64_t>(count, 1) * sizeof(T)));
+  HIP_TRY(device_malloc(&q, std::max<int64_t>(count, 1) * sizeof(T)));
   s->allocations.push_back(q);
   *p = static_cast<T*>(q);
   return CQ35_OK;
@@ -942,7 +968,7 @@ int setup_mega(cq35_session* s) {
   const int64_t final_off = total;
   total += hw;
   void* p = nullptr;
-  HIP_TRY(hipMalloc(&p, total * sizeof(uint64_t)));
+  HIP_TRY(device_malloc(&p, total * sizeof(uint64_t)));
   s->allocations.push_back(p);
   s->words = static_cast<uint64_t*>(p);
   HIP_TRY(hipMemset(s->words, 0, total * sizeof(uint64_t)));
@@ -1014,7 +1040,7 @@ int setup_mega(cq35_session* s) {
     base += layer_tensors(c, l);
   }
   p = nullptr;
-  HIP_TRY(hipMalloc(&p, layers.size() * sizeof(MegaLayer)));
+  HIP_TRY(device_malloc(&p, layers.size() * sizeof(MegaLayer)));
   s->allocations.push_back(p);
   s->d_layers = static_cast<MegaLayer*>(p);
   HIP_TRY(hipMemcpy(s->d_layers, layers.data(), layers.size() * sizeof(MegaLayer), hipMemcpyHostToDevice));
@@ -1042,13 +1068,13 @@ int setup_mega(cq35_session* s) {
   a.spin_limit = 1u << 21;
 #ifdef CQ35_PHASE_TRACE
   p = nullptr;
-  HIP_TRY(hipMalloc(&p, (size_t)grid * kTraceSlots * sizeof(uint64_t)));
+  HIP_TRY(device_malloc(&p, (size_t)grid * kTraceSlots * sizeof(uint64_t)));
   s->allocations.push_back(p);
   a.trace = static_cast<uint64_t*>(p);
 #endif
   if (const char* lim = getenv("CQ35_SPIN_LIMIT")) a.spin_limit = (unsigned)strtoul(lim, nullptr, 10);
   p = nullptr;
-  HIP_TRY(hipMalloc(&p, sizeof(MegaArgs)));
+  HIP_TRY(device_malloc(&p, sizeof(MegaArgs)));
   s->allocations.push_back(p);
   s->d_margs = static_cast<MegaArgs*>(p);
   HIP_TRY(hipMemcpy(s->d_margs, &a, sizeof(MegaArgs), hipMemcpyHostToDevice));
@@ -1117,6 +1143,7 @@ int create_session(cq35_model* m, int64_t capacity, cq35_session** out) {
   check(dalloc(s, &s->attn_scratch, d.Q * (int64_t)s->attn_stride));
   if (rc) { destroy_session(s); return rc; }
   if (const char* g = getenv("CQ35_GRAPH")) s->graph_enabled = atoi(g) != 0;
+  if (const char* g = getenv("CQ35_PREFILL_ROWS")) s->prefill_rows = (std::max(0, std::min(atoi(g), (int)kMChunk)) + 15) / 16 * 16;
   e = hipHostMalloc((void**)&s->h_params, (capacity + 2) * sizeof(uint64_t), hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_best, 2 * sizeof(unsigned long long), hipHostMallocDefault);
   if (e == hipSuccess) e = hipMemset(s->cache, 0, cache_n * sizeof(uint16_t));
@@ -1484,63 +1511,124 @@ hipError_t bgemm_lds_optin() {
   return e;
 }
 
-// Chunk buffers of the batched prefill: kBChunk token rows, or kMChunk when
-// the session has matrix-core components selected at its first multi-token
-// call (their expert weights are then streamed once per kMChunk tokens).
-int setup_prefill(cq35_session* s) {
-  if (s->pf_ready) return CQ35_OK;
+// The projection kernels' LDS, once per model.
+int prefill_kernels(cq35_model* m) {
+  std::call_once(m->prefill_once, [m] { m->prefill_ready = bgemm_lds_optin(); });
+  if (m->prefill_ready != hipSuccess) return fail(CQ35_EDEVICE, "projection kernels' LDS: %s", hipGetErrorString(m->prefill_ready));
+  return CQ35_OK;
+}
+
+// Buffers of one multi-token call, in a block of device_pool: activations of
+// `rows` tokens (a chunk) and the attention scratch.
+struct Prefill {
+  uint16_t *h = nullptr, *x = nullptr, *attn = nullptr;
+  uint16_t *a = nullptr, *b = nullptr, *c = nullptr, *d = nullptr;
+  uint16_t *e = nullptr, *f = nullptr, *g = nullptr, *act = nullptr;
+  float *rope = nullptr, *logits = nullptr, *probs = nullptr, *scratch = nullptr;
+  float *part = nullptr, *spart = nullptr;  // matrix-core experts: routed / shared down sums
+  int *eoff = nullptr, *order = nullptr;    // experts: buckets
+  int* tiles = nullptr;                     // matrix-core experts: tiles that hold work
+  int* ids = nullptr;
+  uint32_t* ranges = nullptr;  // k_bgemm: magnitude ranges of a launch's weight and token tiles
+  int attn_tokens = 0;         // tokens per staged-attention launch (scratch rows)
+  int rows = 0;                // tokens per chunk
+};
+
+// Carve the buffers for chunks of `rows` tokens out of `base` (256-byte
+// aligned pieces). Returns the bytes needed; pointers are only assigned when
+// base != nullptr.
+size_t prefill_layout(const cq35_session* s, int64_t rows, unsigned char* base, Prefill* pf) {
   const Dims& d = s->model->d;
   const cq35_config& c = s->model->cfg;
-  const int64_t VH = c.value_heads, limit = s->matrix ? kMChunk : kBChunk;
-  int64_t m = std::min(limit, (s->capacity + 15) / 16 * 16);
-  // a quarter of the rows where they would take an eighth of what is free
-  const int64_t row_bytes = 2 * (3 * d.H + std::max(d.QKV, 2 * d.QS) + std::max(d.VS, d.KVS) + std::max(2 * VH, d.KVS) +
-                                 std::max(d.QKV, d.QS) + 2 * d.KS + std::max(d.VS, d.QS) + d.VS +
-                                 std::max(d.I, d.K * d.I + d.SI)) + (c.moe ? 4 * ((d.K + 1) * d.H + d.E) : 0);
-  size_t free_bytes = 0, total_bytes = 0;
-  HIP_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
-  if (m * row_bytes > (int64_t)(free_bytes / 8)) m = std::min(m, limit / 4);
-  s->pf_rows = (int)m;
-  int rc = CQ35_OK;
-  auto check = [&](int r) { if (r && !rc) rc = r; };
-  check(dalloc(s, &s->pf_h, m * d.H));
-  check(dalloc(s, &s->pf_x, m * d.H));
-  check(dalloc(s, &s->pf_attn, m * d.H));
-  check(dalloc(s, &s->pf_a, m * std::max(d.QKV, 2 * d.QS)));  // qkv | qg
-  check(dalloc(s, &s->pf_b, m * std::max(d.VS, d.KVS)));      // z | k
-  check(dalloc(s, &s->pf_c, m * std::max(2 * VH, d.KVS)));    // alpha, beta | v
-  check(dalloc(s, &s->pf_d, m * std::max(d.QKV, d.QS)));      // conv | rotated q
-  check(dalloc(s, &s->pf_e, m * 2 * d.KS));                   // l2 q, k
-  check(dalloc(s, &s->pf_f, m * std::max(d.VS, d.QS)));       // core | context
-  check(dalloc(s, &s->pf_g, m * d.VS));                       // gated
-  check(dalloc(s, &s->pf_act, m * std::max(d.I, d.K * d.I + d.SI)));
-  check(dalloc(s, &s->pf_rope, m * std::max<int64_t>(d.R, 2)));
-  check(dalloc(s, &s->pf_ranges, bgemm_range_words(std::max({d.QKV + d.VS + 2 * VH, 2 * d.QS + 2 * d.KVS, d.H, d.I}), m)));
-  if (!rc && bgemm_lds_optin() != hipSuccess) rc = fail(CQ35_EDEVICE, "projection kernels' LDS");
+  const int64_t m = rows, VH = c.value_heads;
+  size_t off = 0;
+  auto take = [&](auto** p, int64_t count) {
+    using T = std::remove_pointer_t<std::remove_reference_t<decltype(p)>>;
+    const size_t bytes = (size_t)std::max<int64_t>(count, 1) * sizeof(std::remove_pointer_t<T>);
+    if (base) *p = reinterpret_cast<T>(base + off);
+    off += (bytes + 255) / 256 * 256;
+  };
+  pf->rows = (int)m;
+  take(&pf->h, m * d.H);
+  take(&pf->x, m * d.H);
+  take(&pf->attn, m * d.H);
+  take(&pf->a, m * std::max(d.QKV, 2 * d.QS));  // qkv | qg
+  take(&pf->b, m * std::max(d.VS, d.KVS));      // z | k
+  take(&pf->c, m * std::max(2 * VH, d.KVS));    // alpha, beta | v
+  take(&pf->d, m * std::max(d.QKV, d.QS));      // conv | rotated q
+  take(&pf->e, m * 2 * d.KS);                   // l2 q, k
+  take(&pf->f, m * std::max(d.VS, d.QS));       // core | context
+  take(&pf->g, m * d.VS);                       // gated
+  take(&pf->act, m * std::max(d.I, d.K * d.I + d.SI));
+  take(&pf->rope, m * std::max<int64_t>(d.R, 2));
+  take(&pf->ranges, bgemm_range_words(std::max({d.QKV + d.VS + 2 * VH, 2 * d.QS + 2 * d.KVS, d.H, d.I}), m));
   if (c.moe) {
-    check(dalloc(s, &s->pf_logits, m * (d.E + 1)));
-    check(dalloc(s, &s->pf_ids, m * d.K));
-    check(dalloc(s, &s->pf_probs, m * d.K));
-    check(dalloc(s, &s->pf_eoff, d.E + 2));
-    check(dalloc(s, &s->pf_order, m * d.K));
-    check(dalloc(s, &s->pf_tiles, 1 + moe_tiles(m, d.K, d.E)));
-    check(dalloc(s, &s->pf_part, m * d.K * d.H));
-    check(dalloc(s, &s->pf_spart, m * d.H));
+    take(&pf->logits, m * (d.E + 1));
+    take(&pf->ids, m * d.K);
+    take(&pf->probs, m * d.K);
+    take(&pf->eoff, d.E + 2);
+    take(&pf->order, m * d.K);
+    take(&pf->tiles, 1 + moe_tiles(m, d.K, d.E));
+    take(&pf->part, m * d.K * d.H);
+    take(&pf->spart, m * d.H);
   }
   // staged attention scratch rows, at most 64 MiB
   const int64_t per_token = d.Q * (int64_t)s->attn_stride;
-  s->pf_attn_tokens = (int)std::max<int64_t>(1, std::min<int64_t>(m, (64ll << 20) / 4 / per_token));
-  check(dalloc(s, &s->pf_scratch, s->pf_attn_tokens * per_token));
-  if (rc) return rc;
-  s->pf_ready = true;
+  pf->attn_tokens = (int)std::max<int64_t>(1, std::min<int64_t>(m, (64ll << 20) / 4 / per_token));
+  take(&pf->scratch, pf->attn_tokens * per_token);
+  return off;
+}
+
+// The block of one call, given back when the call has ended on the device.
+struct PrefillLease {
+  cq35_session* s;
+  DeviceBlock block;
+  Prefill pf;
+  bool ended = false;  // the session's stream has drained
+  explicit PrefillLease(cq35_session* session) : s(session) {}
+  PrefillLease(const PrefillLease&) = delete;
+  ~PrefillLease() {
+    if (!block.p) return;
+    if (ended || hipStreamSynchronize(s->stream) == hipSuccess) device_pool(s->model->device).give(block);
+    else HipMemory::release(block.p);
+  }
+};
+
+// Buffers for a call with the session's components: kBChunk token rows, or
+// kMChunk with matrix-core components (their expert weights are then streamed
+// once per kMChunk tokens), at most the capacity. Where a new block would take
+// an eighth of the free memory or is not to be had, a quarter resp. half of
+// the rows: what is left is for caches, which cannot do with less.
+int prefill_buffers(PrefillLease* lease) {
+  cq35_session* s = lease->s;
+  const int64_t limit = s->prefill_rows ? s->prefill_rows : s->matrix ? kMChunk : kBChunk;
+  const int64_t room = (s->capacity + 15) / 16 * 16;
+  const int64_t rows = std::min(limit, room), few = std::min(s->matrix ? kMFewRows : kBFewRows, rows);
+  auto& pool = device_pool(s->model->device);
+  auto bytes = [&](int64_t m) {
+    Prefill pf;
+    return prefill_layout(s, m, nullptr, &pf);
+  };
+  int64_t m = rows;
+  lease->block = pool.idle(bytes(m));
+  if (!lease->block.p) {
+    size_t free_bytes = 0, total_bytes = 0;
+    HIP_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
+    if (bytes(m) > free_bytes / 8) m = few;
+    if (m < rows) lease->block = pool.idle(bytes(m));
+    if (!lease->block.p) lease->block = pool.allocate(bytes(m));
+    if (!lease->block.p && m > few) lease->block = pool.allocate(bytes(m = few));
+    if (!lease->block.p) return fail(CQ35_EDEVICE, "no device memory for %zu bytes of prompt buffers", bytes(m));
+  }
+  prefill_layout(s, m, static_cast<unsigned char*>(lease->block.p), &lease->pf);
   return CQ35_OK;
 }
 
 // The batched prefill of an n-token call (text-batch, prefill.rs:523-618):
-// shadow import, then per chunk of kBChunk tokens the embedding rows and the
+// shadow import, then per chunk of pf.rows tokens the embedding rows and the
 // layer fold over all rows (batch.full / batch.linear, prefill.rs:92-456),
 // shadow persist, and the head on the call's last row (prefill.row).
-void enqueue_prefill(cq35_session* s, int64_t n) {
+void enqueue_prefill(cq35_session* s, int64_t n, const Prefill& pf) {
   const cq35_model& m = *s->model;
   const cq35_config& c = m.cfg;
   const Dims& d = m.d;
@@ -1551,16 +1639,15 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
   const uint64_t* params = s->d_params;
   enqueue_shadow(s, true);
   int last_rows = 1;
-  // The chunk size changes no result (every per-token operation is
-  // independent of the other rows, the scan carries its state in the shadow),
-  // so the matrix-core components take larger chunks when the buffers allow.
-  const int64_t chunk = s->matrix ? s->pf_rows : std::min<int64_t>(kBChunk, s->pf_rows);
+  // The chunk size changes no result: every per-token operation is
+  // independent of the other rows, the scan carries its state in the shadow.
+  const int64_t chunk = pf.rows;
   for (int64_t c0 = 0; c0 < n; c0 += chunk) {
     const int rows_n = (int)std::min<int64_t>(chunk, n - c0);
     const int first = (int)c0;
     const unsigned tiles = (unsigned)((rows_n + 4 * kBTokens - 1) / (4 * kBTokens));
     L(KC_EMBED, k_bembed, dim3(rows_n), dim3(kBlock), 0, params, first, (const uint16_t*)Wt(0), H,
-      s->pf_h, c0 + rows_n == n ? s->d_best : (unsigned long long*)nullptr);
+      pf.h, c0 + rows_n == n ? s->d_best : (unsigned long long*)nullptr);
     // matrix-core projections when selected (K a multiple of the MFMA step)
     const bool mp = (s->matrix & CQ35_MATRIX_PROJECTIONS) != 0;
     // matrix-core projections: LDS-staged tiles for widths of whole 128-column
@@ -1580,7 +1667,7 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
         return true;
       }
       if (!mp && bgemm_ok(rows_n, cols)) {
-        bgemm<kBPlain>(L, m.cus, x, rows_n, cols, seg, nullptr, nullptr, s->pf_ranges);
+        bgemm<kBPlain>(L, m.cus, x, rows_n, cols, seg, nullptr, nullptr, pf.ranges);
         return true;
       }
       return false;
@@ -1607,7 +1694,7 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
         L(KC_PREFILL_PROJECT, k_mproject<kBResidual>, mgrid(H, cols), dim3(64 * kMWaves), 0, x, rows_n, cols,
           (const uint16_t*)w, (const uint16_t*)nullptr, H, res, out);
       else if (!mp && bgemm_ok(rows_n, cols))
-        bgemm<kBResidual>(L, m.cus, x, rows_n, cols, segments({{w, {out, H}}}), nullptr, res, s->pf_ranges);
+        bgemm<kBResidual>(L, m.cus, x, rows_n, cols, segments({{w, {out, H}}}), nullptr, res, pf.ranges);
       else
         L(KC_PREFILL_PROJECT, k_bproject<kBResidual>,
           dim3((unsigned)((H + bproject_rows<kBResidual>() - 1) / bproject_rows<kBResidual>()), tiles), dim3(kBlock), 0, x,
@@ -1622,21 +1709,21 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
       auto W = [&](int slot) { return Wt(base + slot); };
       const int64_t key_base = l * 2 * cap * d.KVS;
       const int64_t value_base = key_base + cap * d.KVS;
-      norm(s->pf_h, W(0), s->pf_x);
+      norm(pf.h, W(0), pf.x);
       int ffn;
       const void* post_norm;
       if (is_full(c, l)) {
-        uint16_t *qg = s->pf_a, *kraw = s->pf_b, *vraw = s->pf_c, *qr = s->pf_d, *ctx = s->pf_f;
-        if (!project_all(s->pf_x, H, segments({{W(1), {qg, 2 * d.QS}}, {W(2), {kraw, d.KVS}}, {W(3), {vraw, d.KVS}}}))) {
-          project(s->pf_x, H, W(1), (int)(2 * d.QS), qg);
-          project(s->pf_x, H, W(2), (int)d.KVS, kraw);
-          project(s->pf_x, H, W(3), (int)d.KVS, vraw);
+        uint16_t *qg = pf.a, *kraw = pf.b, *vraw = pf.c, *qr = pf.d, *ctx = pf.f;
+        if (!project_all(pf.x, H, segments({{W(1), {qg, 2 * d.QS}}, {W(2), {kraw, d.KVS}}, {W(3), {vraw, d.KVS}}}))) {
+          project(pf.x, H, W(1), (int)(2 * d.QS), qg);
+          project(pf.x, H, W(2), (int)d.KVS, kraw);
+          project(pf.x, H, W(3), (int)d.KVS, vraw);
         }
         L(KC_EMBED, k_brope, dim3(rows_n), dim3(kBlock), 0, params, first, (const float*)m.freq,
-          (int)(d.R / 2), s->pf_rope);
+          (int)(d.R / 2), pf.rope);
         L(KC_PREPARE_FULL, k_full_prepare, dim3((unsigned)(d.Q + d.KVH), rows_n), dim3(kBlock), 0,
           (const uint16_t*)qg, (const uint16_t*)kraw, (const uint16_t*)vraw,
-          (const float*)s->pf_rope, (const float*)W(5), (const float*)W(6), s->cache, key_base,
+          (const float*)pf.rope, (const float*)W(5), (const float*)W(6), s->cache, key_base,
           value_base, params, first, (int)d.KVS, (int)d.Q, (int)d.HD, d.pad_hd, (int)d.R, c.eps, qr, (const SessionRows*)nullptr);
         const float scale = 1.0f / sqrtf((float)d.HD);  // SCALE_BITS, qwen35.rs:701
         auto mattention = [&](auto kernel) {
@@ -1655,30 +1742,30 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
           const int hpk = (int)(d.Q / d.KVH);
           const bool regroup = d.HD % 8 == 0 && d.HD <= 256 && (hpk == 1 || hpk == 2 || hpk == 4 || hpk == 8);
           const int64_t start = (int64_t)s->h_params[0];  // the call's first position
-          for (int a0 = 0; a0 < rows_n; a0 += s->pf_attn_tokens) {
-            const int am = std::min(s->pf_attn_tokens, rows_n - a0);
+          for (int a0 = 0; a0 < rows_n; a0 += pf.attn_tokens) {
+            const int am = std::min(pf.attn_tokens, rows_n - a0);
             const uint16_t* qa = qr + (size_t)a0 * d.QS;
             if (regroup) {
               const unsigned chunks = (unsigned)((start + first + a0 + am + 255) / 256);  // keys of the last token
               if (hpk % 2 == 0)
                 L(KC_ATTENTION, k_bstaged_scores<2>, dim3(chunks, (unsigned)(d.KVH * hpk / 2), (unsigned)am), dim3(256), 0,
                   qa, (const SessionRows*)nullptr, (const uint16_t*)s->cache, params, first + a0, key_base, (int)d.KVS,
-                  (int)d.HD, (int)d.Q, hpk, scale, s->pf_scratch, s->attn_stride);
+                  (int)d.HD, (int)d.Q, hpk, scale, pf.scratch, s->attn_stride);
               else
                 L(KC_ATTENTION, k_bstaged_scores<1>, dim3(chunks, (unsigned)(d.KVH * hpk), (unsigned)am), dim3(256), 0,
                   qa, (const SessionRows*)nullptr, (const uint16_t*)s->cache, params, first + a0, key_base, (int)d.KVS,
-                  (int)d.HD, (int)d.Q, hpk, scale, s->pf_scratch, s->attn_stride);
+                  (int)d.HD, (int)d.Q, hpk, scale, pf.scratch, s->attn_stride);
             }
             L(KC_ATTENTION, k_attention_staged, dim3((unsigned)d.Q, (unsigned)am), dim3(kStagedThreads), 0,
               qa, (const uint16_t*)s->cache, key_base, params,
-              first + a0, (int)d.KVS, (int)d.HD, hpk, scale, s->pf_scratch, s->attn_stride, (const SessionRows*)nullptr,
+              first + a0, (int)d.KVS, (int)d.HD, hpk, scale, pf.scratch, s->attn_stride, (const SessionRows*)nullptr,
               regroup);
             const uint16_t* qga = qg + (size_t)a0 * 2 * d.QS;
             uint16_t* ca = ctx + (size_t)a0 * d.QS;
             const dim3 cgrid((unsigned)(d.KVH * d.HD / kContextChannels), (unsigned)am);
             auto grouped = [&](auto kernel) {
               L(KC_ATTENTION, kernel, cgrid, dim3(kContextThreads), 0, (const uint16_t*)s->cache, params, first + a0,
-                value_base, (int)d.KVS, (int)d.HD, (int)d.Q, qga, (const float*)s->pf_scratch, s->attn_stride, ca,
+                value_base, (int)d.KVS, (int)d.HD, (int)d.Q, qga, (const float*)pf.scratch, s->attn_stride, ca,
                 (const SessionRows*)nullptr);
             };
             if (regroup && hpk == 1) grouped(k_battention_context<1>);
@@ -1688,23 +1775,23 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
             else
               L(KC_ATTENTION, k_attention_context, dim3((unsigned)(d.Q * d.HD / kContextChannels), (unsigned)am),
                 dim3(kContextThreads), 0, (const uint16_t*)s->cache, value_base, params, first + a0, (int)d.KVS,
-                (int)d.HD, (int)d.Q, hpk, qga, (const float*)s->pf_scratch, s->attn_stride, ca,
+                (int)d.HD, (int)d.Q, hpk, qga, (const float*)pf.scratch, s->attn_stride, ca,
                 (const SessionRows*)nullptr);
           }
         }
-        residual_rows(ctx, (int)d.QS, W(4), s->pf_h, s->pf_attn);
+        residual_rows(ctx, (int)d.QS, W(4), pf.h, pf.attn);
         post_norm = W(7);
         ffn = 8;
       } else {
-        uint16_t *qkv = s->pf_a, *z = s->pf_b, *alpha = s->pf_c, *beta = s->pf_c + (size_t)s->pf_rows * VH;
-        uint16_t *conv = s->pf_d, *qn = s->pf_e, *kn = s->pf_e + (size_t)s->pf_rows * d.KS;
-        uint16_t *core = s->pf_f, *gated = s->pf_g;
-        if (!project_all(s->pf_x, H,
+        uint16_t *qkv = pf.a, *z = pf.b, *alpha = pf.c, *beta = pf.c + (size_t)pf.rows * VH;
+        uint16_t *conv = pf.d, *qn = pf.e, *kn = pf.e + (size_t)pf.rows * d.KS;
+        uint16_t *core = pf.f, *gated = pf.g;
+        if (!project_all(pf.x, H,
                          segments({{W(1), {qkv, d.QKV}}, {W(2), {z, d.VS}}, {W(3), {alpha, VH}}, {W(4), {beta, VH}}}))) {
-          project(s->pf_x, H, W(1), (int)d.QKV, qkv);
-          project(s->pf_x, H, W(2), (int)d.VS, z);
-          project(s->pf_x, H, W(3), VH, alpha);
-          project(s->pf_x, H, W(4), VH, beta);
+          project(pf.x, H, W(1), (int)d.QKV, qkv);
+          project(pf.x, H, W(2), (int)d.VS, z);
+          project(pf.x, H, W(3), VH, alpha);
+          project(pf.x, H, W(4), VH, beta);
         }
         const int64_t conv_base = cap * d.KV_STRIDE + l * d.LIN;
         // batched calls have key_dim 128
@@ -1730,18 +1817,18 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
         L(KC_GATED_NORM, k_bgated_norm, dim3((unsigned)((VH * rows_n + gated_rows - 1) / gated_rows)), dim3(kBlock),
           bgated_lds_bytes(c.value_dim), (const uint16_t*)core, (const uint16_t*)z, (const float*)W(7), VH * rows_n,
           gated_rows, c.value_dim, c.eps, gated);
-        residual_rows(gated, (int)d.VS, W(8), s->pf_h, s->pf_attn);
+        residual_rows(gated, (int)d.VS, W(8), pf.h, pf.attn);
         post_norm = W(10);
         ffn = 11;
       }
-      norm(s->pf_attn, post_norm, s->pf_x);
+      norm(pf.attn, post_norm, pf.x);
       if (c.moe) {
         const int E = (int)d.E, K = (int)d.K, I = (int)d.I, SI = (int)d.SI;
         const dim3 rgrid((unsigned)((E + kRouterRows) / kRouterRows),
                          (unsigned)((rows_n + kRouterTokens - 1) / kRouterTokens));
         auto router = [&](auto kernel) {
-          L(KC_ROUTER, kernel, rgrid, dim3(512), 0, (const uint16_t*)s->pf_x, rows_n, (const float*)W(ffn),
-            (const float*)W(ffn + 4), E, s->pf_logits);
+          L(KC_ROUTER, kernel, rgrid, dim3(512), 0, (const uint16_t*)pf.x, rows_n, (const float*)W(ffn),
+            (const float*)W(ffn + 4), E, pf.logits);
         };
         if (H == 2048) router(k_brouter_shared<32>);
         else if (H == 1024) router(k_brouter_shared<16>);
@@ -1749,58 +1836,58 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
         else if (H == 256) router(k_brouter_shared<4>);
         else
           L(KC_ROUTER, k_brouter, dim3((unsigned)((E + 1 + 3) / 4), rows_n), dim3(kBlock), 0,
-            (const uint16_t*)s->pf_x, H, (const float*)W(ffn), (const float*)W(ffn + 4), E,
-            s->pf_logits);
+            (const uint16_t*)pf.x, H, (const float*)W(ffn), (const float*)W(ffn + 4), E,
+            pf.logits);
         L(KC_ROUTER, k_bselect, dim3(rows_n), dim3(kBlock), (size_t)E * 4,
-          (const float*)s->pf_logits, E, K, s->pf_ids, s->pf_probs,
+          (const float*)pf.logits, E, K, pf.ids, pf.probs,
           c0 + rows_n == n ? s->ids + l * d.K : (int*)nullptr);
         const int rows = K * I + SI;
         if ((s->matrix & CQ35_MATRIX_EXPERTS) && H % 16 == 0 && I % 16 == 0 && SI % 16 == 0) {
           L(KC_ROUTER, k_moe_bucket, dim3(1), dim3(1024), (size_t)E * 3 * sizeof(int),
-            (const int*)s->pf_ids, rows_n * K, E, s->pf_eoff, s->pf_order, rows_n, s->pf_tiles);
+            (const int*)pf.ids, rows_n * K, E, pf.eoff, pf.order, rows_n, pf.tiles);
           const int most = moe_tiles(rows_n, K, E);
           const int gate_blocks = (std::max(I, SI) + kXRows - 1) / kXRows, down_blocks = (H + kXRows - 1) / kXRows;
           L(KC_MOE_GATE, k_mmoe_gate, dim3(xtile_grid(gate_blocks, most)),
-            dim3(64 * kXWaves), 0, (const uint16_t*)s->pf_x, H, (const uint16_t*)W(ffn + 1),
+            dim3(64 * kXWaves), 0, (const uint16_t*)pf.x, H, (const uint16_t*)W(ffn + 1),
             (const uint16_t*)W(ffn + 2), (const uint16_t*)W(ffn + 5), (const uint16_t*)W(ffn + 6),
-            (const int*)s->pf_eoff, (const int*)s->pf_order, (const float*)s->pf_probs,
-            (const float*)s->pf_logits, E, K, I, SI, rows_n, (const int*)s->pf_tiles, gate_blocks, s->pf_act);
+            (const int*)pf.eoff, (const int*)pf.order, (const float*)pf.probs,
+            (const float*)pf.logits, E, K, I, SI, rows_n, (const int*)pf.tiles, gate_blocks, pf.act);
           L(KC_MOE_DOWN, k_mmoe_down, dim3(xtile_grid(down_blocks, most)),
-            dim3(64 * kXWaves), 0, (const uint16_t*)s->pf_act, (const uint16_t*)W(ffn + 3),
-            (const uint16_t*)W(ffn + 7), (const int*)s->pf_eoff, (const int*)s->pf_order, E, K, I, SI, H,
-            rows_n, (const int*)s->pf_tiles, down_blocks, s->pf_part, s->pf_spart);
+            dim3(64 * kXWaves), 0, (const uint16_t*)pf.act, (const uint16_t*)W(ffn + 3),
+            (const uint16_t*)W(ffn + 7), (const int*)pf.eoff, (const int*)pf.order, E, K, I, SI, H,
+            rows_n, (const int*)pf.tiles, down_blocks, pf.part, pf.spart);
           L(KC_MOE_DOWN, k_moe_combine, dim3((unsigned)((H + kBlock - 1) / kBlock), (unsigned)rows_n),
-            dim3(kBlock), 0, (const float*)s->pf_part, (const float*)s->pf_spart,
-            (const uint16_t*)s->pf_attn, H, K, s->pf_h);
+            dim3(kBlock), 0, (const float*)pf.part, (const float*)pf.spart,
+            (const uint16_t*)pf.attn, H, K, pf.h);
         } else {
           if (H <= 2048) {
             // the gate/up rows read once per chunk: assignments bucketed by expert
             L(KC_ROUTER, k_moe_bucket, dim3(1), dim3(1024), (size_t)E * 3 * sizeof(int),
-              (const int*)s->pf_ids, rows_n * K, E, s->pf_eoff, s->pf_order, rows_n, (int*)nullptr);
+              (const int*)pf.ids, rows_n * K, E, pf.eoff, pf.order, rows_n, (int*)nullptr);
             auto grouped = [&](auto routed, auto shared) {
               L(KC_MOE_GATE, routed, dim3((unsigned)((I + kGRows - 1) / kGRows), (unsigned)E), dim3(kBlock), 0,
-                (const uint16_t*)s->pf_x, H, (const uint16_t*)W(ffn + 1), (const uint16_t*)W(ffn + 2),
-                (const int*)s->pf_eoff, (const int*)s->pf_order, (const float*)s->pf_probs,
-                (const float*)s->pf_logits, E, K, I, SI, rows_n, s->pf_act);
+                (const uint16_t*)pf.x, H, (const uint16_t*)W(ffn + 1), (const uint16_t*)W(ffn + 2),
+                (const int*)pf.eoff, (const int*)pf.order, (const float*)pf.probs,
+                (const float*)pf.logits, E, K, I, SI, rows_n, pf.act);
               L(KC_MOE_GATE, shared,
                 dim3((unsigned)((SI + kGRows - 1) / kGRows), (unsigned)((rows_n + kGSharedTokens - 1) / kGSharedTokens)),
-                dim3(kBlock), 0, (const uint16_t*)s->pf_x, H, (const uint16_t*)W(ffn + 5),
-                (const uint16_t*)W(ffn + 6), (const int*)s->pf_eoff, (const int*)s->pf_order,
-                (const float*)s->pf_probs, (const float*)s->pf_logits, E, K, I, SI, rows_n, s->pf_act);
+                dim3(kBlock), 0, (const uint16_t*)pf.x, H, (const uint16_t*)W(ffn + 5),
+                (const uint16_t*)W(ffn + 6), (const int*)pf.eoff, (const int*)pf.order,
+                (const float*)pf.probs, (const float*)pf.logits, E, K, I, SI, rows_n, pf.act);
             };
             if (H > 1024) grouped(k_bmoe_gate_grouped<4, false>, k_bmoe_gate_grouped<4, true>);
             else if (H > 512) grouped(k_bmoe_gate_grouped<2, false>, k_bmoe_gate_grouped<2, true>);
             else grouped(k_bmoe_gate_grouped<1, false>, k_bmoe_gate_grouped<1, true>);
           } else {
             L(KC_MOE_GATE, k_bmoe_gate, dim3((unsigned)((rows + 3) / 4), rows_n), dim3(kBlock), 0,
-              (const uint16_t*)s->pf_x, H, (const uint16_t*)W(ffn + 1), (const uint16_t*)W(ffn + 2),
-              (const uint16_t*)W(ffn + 5), (const uint16_t*)W(ffn + 6), (const int*)s->pf_ids,
-              (const float*)s->pf_probs, (const float*)s->pf_logits, E, K, I, SI, s->pf_act);
+              (const uint16_t*)pf.x, H, (const uint16_t*)W(ffn + 1), (const uint16_t*)W(ffn + 2),
+              (const uint16_t*)W(ffn + 5), (const uint16_t*)W(ffn + 6), (const int*)pf.ids,
+              (const float*)pf.probs, (const float*)pf.logits, E, K, I, SI, pf.act);
           }
           auto down_rows = [&](auto kernel) {
             L(KC_MOE_DOWN, kernel, dim3((unsigned)bmoe_down_rows_grid(H, rows_n)), dim3(kBlock), 0,
-              (const uint16_t*)s->pf_act, (const uint16_t*)W(ffn + 3), (const uint16_t*)W(ffn + 7),
-              (const int*)s->pf_ids, (const uint16_t*)s->pf_attn, H, K, I, SI, rows_n, s->pf_h);
+              (const uint16_t*)pf.act, (const uint16_t*)W(ffn + 3), (const uint16_t*)W(ffn + 7),
+              (const int*)pf.ids, (const uint16_t*)pf.attn, H, K, I, SI, rows_n, pf.h);
           };
           const int dq = (K * I / 8 + 63) / 64;  // routed quads per lane
           if (dq <= 1) down_rows(k_bmoe_down_rows<1>);
@@ -1809,27 +1896,27 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
           else if (dq <= 8) down_rows(k_bmoe_down_rows<8>);
           else
             L(KC_MOE_DOWN, k_bmoe_down, dim3((unsigned)bmoe_down_grid(H, rows_n)), dim3(kBlock), 0,
-              (const uint16_t*)s->pf_act, (const uint16_t*)W(ffn + 3), (const uint16_t*)W(ffn + 7),
-              (const int*)s->pf_ids, (const uint16_t*)s->pf_attn, H, K, I, SI, rows_n, s->pf_h);
+              (const uint16_t*)pf.act, (const uint16_t*)W(ffn + 3), (const uint16_t*)W(ffn + 7),
+              (const int*)pf.ids, (const uint16_t*)pf.attn, H, K, I, SI, rows_n, pf.h);
         }
       } else {
         if (mp && H % 16 == 0)
           if (staged(H))
             L(KC_PREFILL_PROJECT, k_mgemm<kBGate>, mgrid((int)d.I, H), dim3(64 * kMWaves), 0,
-              (const uint16_t*)s->pf_x, rows_n, H, segments({{W(ffn), {s->pf_act, d.I}}}),
+              (const uint16_t*)pf.x, rows_n, H, segments({{W(ffn), {pf.act, d.I}}}),
               (const uint16_t*)W(ffn + 1), (const uint16_t*)nullptr);
           else
             L(KC_PREFILL_PROJECT, k_mproject<kBGate>, mgrid((int)d.I, H), dim3(64 * kMWaves), 0,
-              (const uint16_t*)s->pf_x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
-              (int)d.I, (const uint16_t*)nullptr, s->pf_act);
+              (const uint16_t*)pf.x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
+              (int)d.I, (const uint16_t*)nullptr, pf.act);
         else if (!mp && bgemm_ok(rows_n, H))
-          bgemm<kBGate>(L, m.cus, s->pf_x, rows_n, H, segments({{W(ffn), {s->pf_act, d.I}}}), (const uint16_t*)W(ffn + 1),
-                        nullptr, s->pf_ranges);
+          bgemm<kBGate>(L, m.cus, pf.x, rows_n, H, segments({{W(ffn), {pf.act, d.I}}}), (const uint16_t*)W(ffn + 1),
+                        nullptr, pf.ranges);
         else
           L(KC_PREFILL_PROJECT, k_bproject<kBGate>, dim3((unsigned)d.I, tiles), dim3(kBlock), 0,
-            (const uint16_t*)s->pf_x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
-            (int)d.I, (const uint16_t*)nullptr, s->pf_act);
-        residual_rows(s->pf_act, (int)d.I, W(ffn + 2), s->pf_attn, s->pf_h);
+            (const uint16_t*)pf.x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
+            (int)d.I, (const uint16_t*)nullptr, pf.act);
+        residual_rows(pf.act, (int)d.I, W(ffn + 2), pf.attn, pf.h);
       }
       base += layer_tensors(c, l);
     }
@@ -1837,7 +1924,7 @@ void enqueue_prefill(cq35_session* s, int64_t n) {
   }
   enqueue_shadow(s, false);
   const int64_t total = weight_count(c);
-  project32<true>(L, KC_LOGITS, s->pf_h + (size_t)(last_rows - 1) * d.H, (const float*)Wt(total - 2),
+  project32<true>(L, KC_LOGITS, pf.h + (size_t)(last_rows - 1) * d.H, (const float*)Wt(total - 2),
                   c.eps, segments({{Wt(total - 1), {s->logits, d.V}}}), d.H, s->d_best);
 }
 
@@ -2046,10 +2133,11 @@ extern "C" int cq35_session_free(cq35_session* s) {
 namespace {
 
 // Enqueue a validated call on the session's stream (parameter upload, the
-// launches, the token and logits readback), without waiting for it.
-int step_launch(cq35_session* s, const uint64_t* tokens, int64_t n, int64_t start, uint16_t* logits) {
+// launches, the token and logits readback), without waiting for it. `pf`: the
+// buffers of a batched prefill.
+int step_launch(cq35_session* s, const uint64_t* tokens, int64_t n, int64_t start, uint16_t* logits,
+                const Prefill* pf = nullptr) {
   const cq35_config& c = s->model->cfg;
-  const bool batched = n >= 2 && c.key_dim == 128;
   hipError_t e;
   s->h_params[0] = (uint64_t)start;
   for (int64_t i = 0; i < n; ++i) s->h_params[1 + i] = tokens[i];
@@ -2079,8 +2167,8 @@ int step_launch(cq35_session* s, const uint64_t* tokens, int64_t n, int64_t star
     }
     e = hipGraphLaunch(s->graph_exec, s->stream);
     if (e != hipSuccess) return fail(CQ35_EDEVICE, "graph launch: %s", hipGetErrorString(e));
-  } else if (batched) {
-    enqueue_prefill(s, n);
+  } else if (pf) {
+    enqueue_prefill(s, n, *pf);
     e = hipGetLastError();
     if (e != hipSuccess) return fail(CQ35_EDEVICE, "kernel launch: %s", hipGetErrorString(e));
   } else {
@@ -2143,8 +2231,13 @@ extern "C" int cq35_step(cq35_session* s, const uint64_t* tokens, int64_t n, int
   hipError_t e = hipSetDevice(s->model->device);
   if (e != hipSuccess) return fail(CQ35_EDEVICE, "hipSetDevice: %s", hipGetErrorString(e));
   if (batched) {
-    const int rc = setup_prefill(s);
-    if (rc) return rc;
+    PrefillLease lease(s);
+    int rc = prefill_kernels(s->model);
+    if (!rc) rc = prefill_buffers(&lease);
+    if (!rc) rc = step_launch(s, tokens, n, start, logits, &lease.pf);
+    if (!rc) rc = step_complete(s, next_token);
+    lease.ended = rc == CQ35_OK;
+    return rc;
   }
   if (n == 1 && s->mega_on && (s->timed_class < 0 || s->timed_class == KC_DECODE_STEP))
     return step_persistent(s, tokens[0], start, next_token, logits);
@@ -2226,7 +2319,7 @@ int batch_workspace(cq35_model* m, int64_t capacity, int count, BatchWorkspace**
   auto alloc = [&](auto** p, int64_t n) {
     if (e != hipSuccess) return;
     void* q = nullptr;
-    e = hipMalloc(&q, std::max<int64_t>(n, 1) * (int64_t)sizeof(**p));
+    e = device_malloc(&q, std::max<int64_t>(n, 1) * (int64_t)sizeof(**p));
     if (e == hipSuccess) {
       b->allocs.push_back(q);
       *p = static_cast<std::remove_reference_t<decltype(*p)>>(q);

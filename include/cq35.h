@@ -256,10 +256,11 @@ int cq35_session_attention_split(const cq35_session* session, int64_t* keys);
  * expert); bit 2: the full-attention layers' attention over the prompt rows
  * (scores and context on MFMA with the reference's BF16 score, probability
  * and context rounding, qwen35_wmma_attention.hex; head_dim 64, 128 or 256,
- * other head dims keep the exact kernels). 0 keeps the exact SIMT path. A
- * session whose components are set at its first multi-token call runs
- * multi-token calls in chunks of 1024 tokens (otherwise 256; the chunk
- * changes no result). Decode steps (cq35_step with n == 1, and
+ * other head dims keep the exact kernels). 0 keeps the exact SIMT path. Calls
+ * with a component run in chunks of 2048 tokens, others of 1024 (1024 and 256
+ * where device memory is short; the chunk changes no result), in buffers lent
+ * for the length of the call: calls that run at the same time each hold
+ * theirs, sessions between calls none. Decode steps (cq35_step with n == 1, and
  * cq35_step_batch) are unaffected, as the reference's option affects prefill
  * only. */
 #define CQ35_MATRIX_PROJECTIONS 1

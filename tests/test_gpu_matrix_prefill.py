@@ -208,17 +208,15 @@ def test_expert_tiles_cover_every_assignment(name, n):
     assert rel_rms(logits_f32(sm.export_state(0)), logits_f32(se.export_state(0))) <= 0.05
 
 
-def test_matrix_prefill_chunks_same_bits():
-    """2065 tokens over the edge of a 2048-row chunk, against a session whose
-    buffers have the exact path's 1024 rows (its first prompt was exact)."""
+def test_matrix_prefill_chunks_same_bits(monkeypatch):
+    """2065 tokens over the edge of a 2048-row chunk, against chunks of 1024."""
     cfg = shape("mini-moe")
     m = cq35.Model.synthetic(cfg, seed=19)
     prompt = np.random.default_rng(4).integers(0, cfg["vocab"], 2065).tolist()
     components = ALL | Session.MATRIX_ATTENTION
-    one, two = m.session(2080), m.session(2080)
-    two.step_raw(prompt[:2])
-    two.import_state(0, np.zeros_like(two.export_state(0)))
-    two.position = 0
+    one = m.session(2080)
+    monkeypatch.setenv("CQ35_PREFILL_ROWS", "1024")
+    two = m.session(2080)
     one.set_matrix_prefill(components)
     two.set_matrix_prefill(components)
     a, b = one.step_raw(prompt)[0], two.step_raw(prompt)[0]
