@@ -193,17 +193,36 @@ def test_matrix_prefill_switch_leaves_decode_and_exact_path(oracle):
         assert ta == tb and np.array_equal(la, lb)
 
 
-@pytest.mark.parametrize("name,n", [("mini-moe", 2), ("mini-moe", 33), ("mini-moe", 1061), ("qwen36-35b-a3b@4", 65)])
-def test_expert_tiles_cover_every_assignment(name, n):
-    """The listed expert tiles (none, one or several per expert; two, four and
-    sixteen row blocks) against the exact path: an output that no tile writes
-    leaves the 5% gate of the whole prompts above, in the session state."""
-    cfg = shape(name)
+def tile_shape(name):
+    """mini-moe with hidden H, experts of I columns, a shared one of SI, E
+    experts: 'H-I-SI-E'; else a preset."""
+    if name.count("-") != 3 or not name[0].isdigit():
+        return shape(name)
+    cfg = cc.preset("mini-moe")
+    cfg.update(zip(("hidden", "intermediate", "shared_intermediate", "experts"), map(int, name.split("-"))))
+    return cfg
+
+
+@pytest.mark.parametrize("name,n", [
+    ("mini-moe", 2), ("mini-moe", 33), ("mini-moe", 1061), ("qwen36-35b-a3b@4", 65), ("qwen36-35b-a3b@4", 1061),
+    ("1024-384-128-72", 257), ("1536-128-128-200", 300), ("384-256-640-32", 100)])
+def test_expert_tiles_cover_every_assignment(monkeypatch, name, n):
+    """The listed expert tiles (none, one or several per expert, expert counts
+    that are no multiple of a wave; one, two, three, four, five, eight, twelve
+    and sixteen row blocks) against the same prompt in chunks of 16 tokens,
+    where every expert has one tile at most, bit for bit: logits and the whole
+    session state. An output row that no tile writes, or another's tile wrote,
+    shows in it. And against the exact path, within the 5% gate of the whole
+    prompts above."""
+    cfg = tile_shape(name)
     say("expert tiles", name, n)
     m = cq35.Model.synthetic(cfg, seed=23)
     prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).tolist()
     se, ce = prefill(m, prompt, 0, n + 8)
     sm, cm = prefill(m, prompt, Session.MATRIX_EXPERTS, n + 8)
+    monkeypatch.setenv("CQ35_PREFILL_ROWS", "16")
+    ss, cs = prefill(m, prompt, Session.MATRIX_EXPERTS, n + 8)
+    assert np.array_equal(cm[0][1], cs[0][1]) and np.array_equal(sm.export_state(0), ss.export_state(0))
     assert rel_rms(logits_f32(cm[0][1]), logits_f32(ce[0][1])) <= 0.05
     assert rel_rms(logits_f32(sm.export_state(0)), logits_f32(se.export_state(0))) <= 0.05
 
