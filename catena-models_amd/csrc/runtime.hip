@@ -1468,8 +1468,14 @@ const char* prefill_unsupported(const cq35_model& m) {
 // The exact projections of n token rows on the matrix cores (k_bgemm, then
 // k_bgemm_fix): widths of whole 128-byte lines, eight tokens or more. Below,
 // k_bproject: a tile's sixteen columns would be mostly empty (four 2B layers,
-// whole call, at 5 / 8 tokens: 871 / 1073 us against 916 / 923 here).
-bool bgemm_ok(int n, int64_t cols) { return cols % 64 == 0 && n >= kBTokens; }
+// whole call, at 5 / 8 tokens: 871 / 1073 us against 916 / 923 here). Weights
+// at 16-byte addresses, which their loads into LDS ask for (a caller's own
+// device tensors may lie elsewhere; the vector kernel's loads take any).
+bool bgemm_ok(int n, int64_t cols, std::initializer_list<const void*> weights) {
+  uintptr_t address = 0;
+  for (const void* w : weights) address |= (uintptr_t)w;
+  return cols % 64 == 0 && n >= kBTokens && address % 16 == 0;
+}
 
 template <int kMode, int TT, int RT, typename Launch>
 void bgemm_launch(Launch& L, int cus, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2,
@@ -1666,7 +1672,7 @@ void enqueue_prefill(cq35_session* s, int64_t n, const Prefill& pf) {
           rows_n, cols, seg, (const uint16_t*)nullptr, (const uint16_t*)nullptr);
         return true;
       }
-      if (!mp && bgemm_ok(rows_n, cols)) {
+      if (!mp && bgemm_ok(rows_n, cols, {seg.w[0], seg.w[1], seg.w[2], seg.w[3]})) {
         bgemm<kBPlain>(L, m.cus, x, rows_n, cols, seg, nullptr, nullptr, pf.ranges);
         return true;
       }
@@ -1693,7 +1699,7 @@ void enqueue_prefill(cq35_session* s, int64_t n, const Prefill& pf) {
       else if (mp && cols % 16 == 0)
         L(KC_PREFILL_PROJECT, k_mproject<kBResidual>, mgrid(H, cols), dim3(64 * kMWaves), 0, x, rows_n, cols,
           (const uint16_t*)w, (const uint16_t*)nullptr, H, res, out);
-      else if (!mp && bgemm_ok(rows_n, cols))
+      else if (!mp && bgemm_ok(rows_n, cols, {w}))
         bgemm<kBResidual>(L, m.cus, x, rows_n, cols, segments({{w, {out, H}}}), nullptr, res, pf.ranges);
       else
         L(KC_PREFILL_PROJECT, k_bproject<kBResidual>,
@@ -1909,7 +1915,7 @@ void enqueue_prefill(cq35_session* s, int64_t n, const Prefill& pf) {
             L(KC_PREFILL_PROJECT, k_mproject<kBGate>, mgrid((int)d.I, H), dim3(64 * kMWaves), 0,
               (const uint16_t*)pf.x, rows_n, H, (const uint16_t*)W(ffn), (const uint16_t*)W(ffn + 1),
               (int)d.I, (const uint16_t*)nullptr, pf.act);
-        else if (!mp && bgemm_ok(rows_n, H))
+        else if (!mp && bgemm_ok(rows_n, H, {W(ffn), W(ffn + 1)}))
           bgemm<kBGate>(L, m.cus, pf.x, rows_n, H, segments({{W(ffn), {pf.act, d.I}}}), (const uint16_t*)W(ffn + 1),
                         nullptr, pf.ranges);
         else
@@ -3089,7 +3095,7 @@ template <int kMode>
 void device_exact_gemm(int route, int cus, const uint16_t* x, int n, int cols, const uint16_t* w, const uint16_t* w2,
                        int rows, const uint16_t* res, uint16_t* out, uint32_t* ranges) {
   DirectLauncher L;
-  if (route == 1 && bgemm_ok(n, cols)) {
+  if (route == 1 && bgemm_ok(n, cols, {w, w2})) {
     bgemm<kMode>(L, cus, x, n, cols, segments({{w, {out, rows}}}), w2, res, ranges);
     return;
   }

@@ -17,6 +17,7 @@ import time
 
 import numpy as np
 import pytest
+import torch
 
 import cq35
 import cq35.config as cc
@@ -293,3 +294,27 @@ def test_inexact_tiles_cost_no_cliff(oracle):
     ordinary = seconds(plain, "none")
     assert seconds(with_tiny(slice(3, 4)), "one row tile per matrix") < 6 * ordinary
     assert seconds(with_tiny(slice(0, None, 8)), "all") < 6 * ordinary
+
+
+def test_borrowed_weights_off_the_lds_alignment(oracle):
+    """Weights that a caller placed at addresses of 8 modulo 16: the same
+    prompt as with the library's own, bit for bit (the vector kernel's loads
+    take any address; the loads into LDS ask for 16 bytes)."""
+    cfg = config(576, 1344)
+    weights = oracle.synthetic_weights(cfg, 33)
+    tensors = []
+    for w in weights:
+        t = torch.empty(w.nbytes + 64, dtype=torch.uint8, device="cuda")
+        at = 8 - t.data_ptr() % 16 + 16
+        t[at:at + w.nbytes] = torch.from_numpy(np.ascontiguousarray(w).view(np.uint8)).cuda()
+        tensors.append((t, at))
+    torch.cuda.synchronize()
+    pointers = (ctypes.c_void_p * len(weights))(*[t.data_ptr() + at for t, at in tensors])
+    c, handle = cc.to_c(cfg), ctypes.c_void_p()
+    _lib.check(_lib.load().cq35_model_create(ctypes.byref(c), pointers, 1, ctypes.byref(handle)))
+    borrowed, own = cq35.Model(handle.value, cfg), cq35.Model.from_arrays(cfg, weights)
+    prompt = np.random.default_rng(2).integers(0, cfg["vocab"], 70).tolist()
+    print("borrowed weights", flush=True)
+    a, b = borrowed.session(70), own.session(70)
+    (la, ta), (lb, tb) = a.step_raw(prompt), b.step_raw(prompt)
+    assert ta == tb and np.array_equal(la, lb) and np.array_equal(a.export_state(0), b.export_state(0))
