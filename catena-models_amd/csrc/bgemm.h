@@ -45,18 +45,18 @@ namespace cq35 {
 constexpr int kEWaves = 8;
 constexpr int kEThreads = 64 * kEWaves;
 
-// Token tiles and weight-row tiles of 16 per block.
-template <int TT, int RT>
+// Token tiles of 16 per block, by one of 16 weight rows.
+template <int TT>
 struct BGemmTile {
-  static constexpr int kTiles = TT * RT, kTokens = 16 * TT, kRows = 16 * RT, kStaged = kTokens + kRows;
-  static constexpr int kOut = 256 * kTiles;        // outputs per block
+  static constexpr int kTokens = 16 * TT, kRows = 16, kStaged = kTokens + kRows;
+  static constexpr int kOut = 256 * TT;            // outputs per block
   static constexpr int kStage = kStaged * 16;      // 16-byte pieces per stage (two lines per row)
   static constexpr int kLoads = (kStage + kEThreads - 1) / kEThreads;
   // the waves' sums: 4 lanes of the quad x kOut F32 each
   static constexpr size_t kSums = (size_t)kEWaves * 4 * kOut * 4;
   static constexpr int kBufs = 4;  // LDS stages: one read, the others on their way
   static constexpr size_t kLds = kSums + kBufs * (size_t)kStage * 16;
-  static constexpr int kBlocksPerCu = kTiles == 1 ? 2 : 1;
+  static constexpr int kBlocksPerCu = TT == 1 ? 2 : 1;
 };
 
 // What a piece past the end of a row reads.
@@ -110,8 +110,8 @@ __device__ __forceinline__ uint32_t range_of(const uint32_t* ranges, int tile) {
 
 // Output rows per block: in gate mode a tile holds eight gate rows and the
 // same eight up rows.
-template <int kMode, int RT>
-constexpr int bgemm_rows() { return kMode == kBGate ? 8 * RT : 16 * RT; }
+template <int kMode>
+constexpr int bgemm_rows() { return kMode == kBGate ? 8 : 16; }
 
 // out_s[t][r] of n token rows against the concatenated rows of `seg` (gate
 // mode: one segment, w2 the up matrix), k_bproject's epilogues. cols % 64 ==
@@ -120,13 +120,13 @@ constexpr int bgemm_rows() { return kMode == kBGate ? 8 * RT : 16 * RT; }
 // row tiles = b mod 8: a row tile's token tiles follow each other there, so a
 // weight tile comes from HBM once. `ranges`: kEWaves words per row tile, then
 // per token tile.
-template <int kMode, int TT, int RT>
-__global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) void k_bgemm(const uint16_t* __restrict__ x, int n, int cols, Segments seg,
+template <int kMode, int TT>
+__global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT>::kBlocksPerCu)) void k_bgemm(const uint16_t* __restrict__ x, int n, int cols, Segments seg,
                                                      const uint16_t* __restrict__ w2,
                                                      const uint16_t* __restrict__ res,
                                                      uint32_t* __restrict__ ranges) {
-  using T = BGemmTile<TT, RT>;
-  constexpr int NT = T::kTiles, kBlockRows = bgemm_rows<kMode, RT>();
+  using T = BGemmTile<TT>;
+  constexpr int kBlockRows = bgemm_rows<kMode>();
   extern __shared__ __align__(16) u32x4 bg_lds[];
   f32x4* sums = reinterpret_cast<f32x4*>(bg_lds);
   u32x4* stage = bg_lds + T::kSums / 16;
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
       } else {
         int wr = row - T::kTokens;
         const bool up = kMode == kBGate && (wr & 8) != 0;
-        if (kMode == kBGate) wr = (wr >> 4) * 8 + (wr & 7);
+        if (kMode == kBGate) wr &= 7;
         int local;
         const int s = segment_of(seg, min(r0 + wr, rows - 1), &local);
         base = (up ? w2 : segment_w(seg, s)) + (size_t)local * cols;
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
       if (weights) {
         const bool up = kMode == kBGate && (row & 8) != 0;
         int local;
-        const int s = segment_of(seg, min(row0 + (kMode == kBGate ? (row >> 4) * 8 + (row & 7) : row), rows - 1), &local);
+        const int s = segment_of(seg, min(row0 + (kMode == kBGate ? row & 7 : row), rows - 1), &local);
         base = (up ? w2 : segment_w(seg, s)) + (size_t)local * cols;
       } else {
         base = x + (size_t)min(row0 + row, n - 1) * cols;
@@ -251,48 +251,35 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
   const int i16 = lane & 15, visit = lane >> 5;
   const uint32_t half = (lane >> 4) & 1 ? 0x03020c0cu : 0x01000c0cu;
   const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  f32x4 a0[4][NT], a1[4][NT], a2[4][NT];  // lines' sums
-  u32x4 a[TT], b[RT];
-  float a3[TT], b3[RT];
+  f32x4 a0[4][TT], a1[4][TT], a2[4][TT];  // lines' sums
+  u32x4 a[TT], b;
+  float a3[TT], b3;
   auto read = [&](int buf) {
     const u32x4* s = stage + buf * T::kStage;
     auto piece = [&](int row) { return s[(row * 2 + visit) * 8 + (c ^ (row & 7))]; };
 #pragma unroll
     for (int t = 0; t < TT; ++t) a[t] = piece(16 * t + i16);
-#pragma unroll
-    for (int r = 0; r < RT; ++r) b[r] = piece(T::kTokens + 16 * r + i16);
+    b = piece(T::kTokens + i16);
   };
-  auto multiply = [&](f32x4 (&acc)[4][NT], auto first) {
+  auto multiply = [&](f32x4 (&acc)[4][TT], auto first) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      float af[TT], bf[RT];
+      float af[TT];
 #pragma unroll
       for (int t = 0; t < TT; ++t) af[t] = bitsf(__builtin_amdgcn_perm(0u, a[t][j], half));
+      const float bf = bitsf(__builtin_amdgcn_perm(0u, b[j], half));
 #pragma unroll
-      for (int r = 0; r < RT; ++r) bf[r] = bitsf(__builtin_amdgcn_perm(0u, b[r][j], half));
-#pragma unroll
-      for (int t = 0; t < TT; ++t)
-#pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          if (j == 3) continue;
-          acc[j][t * RT + r] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              af[t], bf[r], decltype(first)::value ? zero : acc[j][t * RT + r], 0, 0, 0);
-        }
-      if (j == 3) {
-#pragma unroll
-        for (int t = 0; t < TT; ++t) a3[t] = af[t];
-#pragma unroll
-        for (int r = 0; r < RT; ++r) b3[r] = bf[r];
+      for (int t = 0; t < TT; ++t) {
+        if (j == 3) a3[t] = af[t];
+        else acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[t], bf, decltype(first)::value ? zero : acc[j][t], 0, 0, 0);
       }
+      if (j == 3) b3 = bf;
     }
   };
-  auto last_lane = [&](f32x4 (&acc)[4][NT], auto first) {
+  auto last_lane = [&](f32x4 (&acc)[4][TT], auto first) {
 #pragma unroll
     for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int r = 0; r < RT; ++r)
-        acc[3][t * RT + r] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-            a3[t], b3[r], decltype(first)::value ? zero : acc[3][t * RT + r], 0, 0, 0);
+      acc[3][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a3[t], b3, decltype(first)::value ? zero : acc[3][t], 0, 0, 0);
   };
 
   static_assert(T::kStage % kEThreads == 0 && T::kBufs >= 2, "requests per stage");
@@ -301,15 +288,15 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
 #pragma unroll 1
   for (int i = 0; i < T::kBufs - 1; ++i) fetch();
   arrived();
-  f32x4* mine = sums + (size_t)c * 4 * NT * 64;  // [j][tile][lane]
+  f32x4* mine = sums + (size_t)c * 4 * TT * 64;  // [j][tile][lane]
   // what becomes of the sums when a line is done, lanes j0 .. j1 - 1: a half's
   // lines 0 and 1 go to a0 and a1 (a0 += a1), 2 and 3 to a1 and a2
   auto fold = [&](auto k, int j0, int j1) {
 #pragma unroll
     for (int j = j0; j < j1; ++j)
 #pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        f32x4* m = &mine[(j * NT + i) * 64 + lane];
+      for (int i = 0; i < TT; ++i) {
+        f32x4* m = &mine[(j * TT + i) * 64 + lane];
         if (k() == 1) a0[j][i] = a0[j][i] + a1[j][i];
         if (k() == 3) *m = a0[j][i] + (a1[j][i] + a2[j][i]);
         if (k() == 4) *m = *m + (a0[j][i] + (a1[j][i] + a2[j][i]));
@@ -317,7 +304,7 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
   };
   // the last products of line k of a half (4: of the second half's line 3)
   auto finish_line = [&](auto k) {
-    f32x4(&acc)[4][NT] = k() == 0 ? a0 : k() < 3 ? a1 : a2;
+    f32x4(&acc)[4][TT] = k() == 0 ? a0 : k() < 3 ? a1 : a2;
     fold(k, 0, 3);
     if (pairs == 1) last_lane(acc, std::true_type{});
     else last_lane(acc, std::false_type{});
@@ -335,7 +322,7 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
     for (int h = 0; h < 2; ++h) {
       // line k's chains
       auto run_line = [&](auto k) {
-        f32x4(&acc)[4][NT] = k() == 0 ? a0 : k() < 3 ? a1 : a2;
+        f32x4(&acc)[4][TT] = k() == 0 ? a0 : k() < 3 ? a1 : a2;
         auto one = [&](int sp, auto first) {
           if (decltype(first)::value) {
             if (k() != 0) finish_line(std::integral_constant<int, (decltype(k)::value + 3) % 4>{});
@@ -374,18 +361,18 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
       for (int j = 0; j < 4; ++j) {
         float p[kEWaves];
 #pragma unroll
-        for (int w = 0; w < kEWaves; ++w) p[w] = f[((w * 4 + j) * NT + tile) * 256 + o];
+        for (int w = 0; w < kEWaves; ++w) p[w] = f[((w * 4 + j) * TT + tile) * 256 + o];
         v[j] = ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
       }
       return (v[0] + v[2]) + (v[1] + v[3]);
     };
     // gate mode: rows 0-7 of a tile are gate rows, 8-15 the same up rows
-    for (int i = tid_here(); i < 256 * NT; i += kEThreads) {
-      const int tile = i >> 8, o = i & 255, tt = tile / RT, rt = tile - tt * RT, col = (o >> 2) & 15;
+    for (int i = tid_here(); i < 256 * TT; i += kEThreads) {
+      const int tile = i >> 8, o = i & 255, col = (o >> 2) & 15;
       if (kMode == kBGate && col >= 8) continue;
       const float v = total(tile, o);
       const float v2 = kMode == kBGate ? total(tile, o + 32) : 0.0f;
-      const int t = t0 + 16 * tt + 4 * (o >> 6) + (o & 3), r = r0 + (kMode == kBGate ? 8 : 16) * rt + col;
+      const int t = t0 + 16 * tile + 4 * (o >> 6) + (o & 3), r = r0 + col;
       if (t < n && r < rows) {
         int local;
         const int s = segment_of(seg, r, &local);
@@ -412,13 +399,13 @@ __global__ __launch_bounds__(kEThreads, (2 * BGemmTile<TT, RT>::kBlocksPerCu)) v
 // exact (one block per 256 tiles, recomputing alone: 118 and 1510).
 constexpr int kFixThreads = 1024, kFixGroups = kFixThreads / 256;
 
-template <int kMode, int TT, int RT>
+template <int kMode, int TT>
 __global__ __launch_bounds__(kFixThreads) void k_bgemm_fix(const uint16_t* __restrict__ x, int n, int cols, Segments seg,
                                                            const uint16_t* __restrict__ w2,
                                                            const uint16_t* __restrict__ res,
                                                            const uint32_t* __restrict__ ranges) {
-  using T = BGemmTile<TT, RT>;
-  constexpr int kBlockRows = bgemm_rows<kMode, RT>(), R = bproject_rows<kMode>();
+  using T = BGemmTile<TT>;
+  constexpr int kBlockRows = bgemm_rows<kMode>(), R = bproject_rows<kMode>();
   static_assert(kBlockRows % R == 0 && T::kTokens % kBTokens == 0, "a region lies in one tile");
   const int rows = seg.rows[0] + seg.rows[1] + seg.rows[2] + seg.rows[3];
   const int tiles_t = (n + T::kTokens - 1) / T::kTokens, tiles_r = (rows + kBlockRows - 1) / kBlockRows;

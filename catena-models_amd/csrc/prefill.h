@@ -21,6 +21,7 @@
 namespace cq35 {
 
 constexpr int kBTokens = 8;   // tokens per wave sharing each weight quad
+constexpr int kBKeyDim = 128;  // DeltaNet key width of batched calls (others run token by token)
 // Tokens per chunk (buffer rows), exact and with matrix-core components: each
 // chunk streams every weight once, expert weights above all (1.6 GB a 35B
 // layer), and a short last chunk fills few tiles. Eight layers, whole call:
@@ -207,13 +208,13 @@ __global__ __launch_bounds__(kBlock) void k_bnorm(const uint16_t* __restrict__ x
 // tokens in turn would be the time (37 tokens: 6 us, 10 at TB 32).
 constexpr int kPrepareTokens = 32, kPrepareFew = 8;
 
-template <int KD, int TB>
+template <int TB>
 __global__ __launch_bounds__(kBlock) void k_bprepare(
     const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ cache, int64_t conv_base,
     const uint64_t* __restrict__ params, int first, int m, const float* __restrict__ conv_w, int qkv_size,
     int key_heads, uint16_t* __restrict__ conv_out, uint16_t* __restrict__ q_out,
     uint16_t* __restrict__ k_out) {
-  constexpr int kPairs = KD / 2, kGroups = kBlock / kPairs, kEach = TB / kGroups;
+  constexpr int KD = kBKeyDim, kPairs = KD / 2, kGroups = kBlock / kPairs, kEach = TB / kGroups;
   static_assert(kBlock % kPairs == 0 && TB % kGroups == 0, "channel pairs");
   __shared__ float squares[TB][KD + 1];
   __shared__ float total[TB];
@@ -361,7 +362,7 @@ __device__ __forceinline__ float sum32_everywhere(float v) {
 // (batch.scan, batch_scan.hex:1-200): per token exactly the single-step
 // arithmetic of k_delta (32 lanes per value channel, lane l owns key elements
 // l, l+32, ...; serial from 0.0, 32-wide halving tree), 8 channels of one head
-// per block. Requires key_dim <= 256 and value_dim % 8 == 0.
+// per block. Requires value_dim % 8 == 0.
 //
 // Bound: instruction issue of a token's serial chain (two sums over 32
 // reference lanes, the state update between them). The chain holds nothing
@@ -376,21 +377,18 @@ __device__ __forceinline__ float sum32_everywhere(float v) {
 // wave per SIMD: 218).
 constexpr int kScanTokens = 32;
 
-__host__ __device__ constexpr size_t bscan_lds_bytes(int key_dim) {
-  return (size_t)kScanTokens * key_dim * 2 * 4 + (size_t)kScanTokens * 8 + (size_t)kScanTokens * 8 * (4 + 2);
-}
+constexpr size_t kScanLds = (size_t)kScanTokens * kBKeyDim * 2 * 4 + (size_t)kScanTokens * 8 + (size_t)kScanTokens * 8 * (4 + 2);
 
-template <int KJ>  // key elements per lane: key_dim / 32
 __global__ __launch_bounds__(kBlock) void k_bscan(
     const uint16_t* __restrict__ conv, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ alpha,
     const uint16_t* __restrict__ beta, const float* __restrict__ dt, const float* __restrict__ a,
     float* __restrict__ state, int m, int value_size, int value_dim, int value_heads, int key_heads, int qkv_size,
     float scale, uint16_t* __restrict__ out) {
-  constexpr int key_dim = 32 * KJ, quads = key_dim / 8;
+  constexpr int key_dim = kBKeyDim, KJ = key_dim / 32, quads = key_dim / 8;  // KJ key elements per lane
   constexpr int CH = kBlock / 32;  // channels
   constexpr int kRows = kScanTokens * quads / kBlock;  // quads of k and of q per thread and stage
-  static_assert(kScanTokens == 32 && kScanTokens * CH == kBlock, "a token per lane, a value per thread");
+  static_assert(kScanTokens == 32 && kScanTokens * CH == kBlock && kRows * kBlock == kScanTokens * quads, "a token per lane, a value per thread");
   extern __shared__ __align__(16) unsigned char scan_lds[];
   float* sk = reinterpret_cast<float*>(scan_lds);
   float* sq = sk + kScanTokens * key_dim;
@@ -408,14 +406,14 @@ __global__ __launch_bounds__(kBlock) void k_bscan(
   float s[KJ];
 #pragma unroll
   for (int j = 0; j < KJ; ++j) s[j] = state[(size_t)c * key_dim + lane + 32 * j];
-  u32x4 kq4[kRows > 0 ? kRows : 1], qq4[kRows > 0 ? kRows : 1];
+  u32x4 kq4[kRows], qq4[kRows];
   uint16_t val, al, be;
   // a stage's rows into registers (rows past the last repeat it)
   auto request = [&](int t0) {
 #pragma unroll
-    for (int r = 0; r < (kRows > 0 ? kRows : 1); ++r) {
+    for (int r = 0; r < kRows; ++r) {
       const int idx = threadIdx.x + kBlock * r;
-      const int t = min(t0 + min(idx / quads, kScanTokens - 1), m - 1);
+      const int t = min(t0 + idx / quads, m - 1);
       const size_t src = (size_t)t * key_size + kbase + 8 * (idx % quads);
       kq4[r] = *reinterpret_cast<const u32x4*>(k + src);
       qq4[r] = *reinterpret_cast<const u32x4*>(q + src);
@@ -427,9 +425,8 @@ __global__ __launch_bounds__(kBlock) void k_bscan(
   };
   auto place = [&]() {
 #pragma unroll
-    for (int r = 0; r < (kRows > 0 ? kRows : 1); ++r) {
+    for (int r = 0; r < kRows; ++r) {
       const int idx = threadIdx.x + kBlock * r;
-      if (idx >= kScanTokens * quads) continue;
       auto widen = [&](float* to, const u32x4& v) {
         f32x4* d = reinterpret_cast<f32x4*>(to + 8 * idx);
         d[0] = f32x4{lo2f(v.x), hi2f(v.x), lo2f(v.y), hi2f(v.y)};

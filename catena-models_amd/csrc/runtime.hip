@@ -1453,11 +1453,8 @@ const char* prefill_unsupported(const cq35_model& m) {
   const Dims& d = m.d;
   const cq35_config& c = m.cfg;
   if (d.H % 8 || d.QS % 8 || d.VS % 8) return "hidden, query and value widths must be multiples of 8";
-  if (c.key_dim > 256) return "key_dim above 256";
-  if (c.key_dim != 32 && c.key_dim != 64 && c.key_dim != 128 && c.key_dim != 256)
-    return "key_dim must be 32, 64, 128 or 256";
+  if (c.key_dim != kBKeyDim) return "key_dim must be 128";
   if (c.value_dim % 8) return "value_dim must be a multiple of 8 (eight channels of one head per scan block)";
-  if (bscan_lds_bytes(c.key_dim) > 65536) return "key_dim too large for the scan's LDS stage";
   if (d.I % 8) return "intermediate width must be a multiple of 8";
   if (c.moe && (d.SI % 8 || d.SI > d.K * d.I))
     return "shared-expert width must be a multiple of 8 and at most top_k * intermediate";
@@ -1477,16 +1474,16 @@ bool bgemm_ok(int n, int64_t cols, std::initializer_list<const void*> weights) {
   return cols % 64 == 0 && n >= kBTokens && address % 16 == 0;
 }
 
-template <int kMode, int TT, int RT, typename Launch>
+template <int kMode, int TT, typename Launch>
 void bgemm_launch(Launch& L, int cus, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2,
                   const uint16_t* res, uint32_t* ranges) {
-  using T = BGemmTile<TT, RT>;
-  const int per = bgemm_rows<kMode, RT>();
+  using T = BGemmTile<TT>;
+  const int per = bgemm_rows<kMode>();
   const int tr = (int)((seg_rows(seg) + per - 1) / per), tt = (n + T::kTokens - 1) / T::kTokens;
   const int grid = std::min((tr + 7) / 8 * tt, std::max(cus / 8, 1) * T::kBlocksPerCu) * 8;
-  L(KC_PREFILL_PROJECT, k_bgemm<kMode, TT, RT>, dim3((unsigned)grid), dim3(kEThreads), T::kLds, x, n, cols, seg, w2, res,
+  L(KC_PREFILL_PROJECT, k_bgemm<kMode, TT>, dim3((unsigned)grid), dim3(kEThreads), T::kLds, x, n, cols, seg, w2, res,
     ranges);
-  L(KC_PREFILL_PROJECT, k_bgemm_fix<kMode, TT, RT>, dim3((unsigned)cus), dim3(kFixThreads), 0, x, n, cols, seg, w2,
+  L(KC_PREFILL_PROJECT, k_bgemm_fix<kMode, TT>, dim3((unsigned)cus), dim3(kFixThreads), 0, x, n, cols, seg, w2,
     res, (const uint32_t*)ranges);
 }
 
@@ -1498,8 +1495,8 @@ void bgemm_launch(Launch& L, int cus, const uint16_t* x, int n, int cols, const 
 template <int kMode, typename Launch>
 void bgemm(Launch& L, int cus, const uint16_t* x, int n, int cols, const Segments& seg, const uint16_t* w2,
            const uint16_t* res, uint32_t* ranges) {
-  if (n <= (kMode == kBGate ? 32 : 256)) bgemm_launch<kMode, 1, 1>(L, cus, x, n, cols, seg, w2, res, ranges);
-  else bgemm_launch<kMode, 3, 1>(L, cus, x, n, cols, seg, w2, res, ranges);
+  if (n <= (kMode == kBGate ? 32 : 256)) bgemm_launch<kMode, 1>(L, cus, x, n, cols, seg, w2, res, ranges);
+  else bgemm_launch<kMode, 3>(L, cus, x, n, cols, seg, w2, res, ranges);
 }
 
 // Words of k_bgemm's ranges for launches of at most `rows` rows and n tokens:
@@ -1508,9 +1505,9 @@ int64_t bgemm_range_words(int64_t rows, int64_t n) { return rows + n + 2 * 8 * k
 
 hipError_t bgemm_lds_optin() {
   const std::pair<const void*, size_t> f[] = {
-      {(const void*)k_bgemm<kBPlain, 1, 1>, BGemmTile<1, 1>::kLds}, {(const void*)k_bgemm<kBPlain, 3, 1>, BGemmTile<3, 1>::kLds},
-      {(const void*)k_bgemm<kBResidual, 1, 1>, BGemmTile<1, 1>::kLds}, {(const void*)k_bgemm<kBResidual, 3, 1>, BGemmTile<3, 1>::kLds},
-      {(const void*)k_bgemm<kBGate, 1, 1>, BGemmTile<1, 1>::kLds}, {(const void*)k_bgemm<kBGate, 3, 1>, BGemmTile<3, 1>::kLds}};
+      {(const void*)k_bgemm<kBPlain, 1>, BGemmTile<1>::kLds}, {(const void*)k_bgemm<kBPlain, 3>, BGemmTile<3>::kLds},
+      {(const void*)k_bgemm<kBResidual, 1>, BGemmTile<1>::kLds}, {(const void*)k_bgemm<kBResidual, 3>, BGemmTile<3>::kLds},
+      {(const void*)k_bgemm<kBGate, 1>, BGemmTile<1>::kLds}, {(const void*)k_bgemm<kBGate, 3>, BGemmTile<3>::kLds}};
   hipError_t e = hipSuccess;
   for (const auto& k : f)
     if (e == hipSuccess) e = hipFuncSetAttribute(k.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.second);
@@ -1800,22 +1797,17 @@ void enqueue_prefill(cq35_session* s, int64_t n, const Prefill& pf) {
           project(pf.x, H, W(4), VH, beta);
         }
         const int64_t conv_base = cap * d.KV_STRIDE + l * d.LIN;
-        // batched calls have key_dim 128
         const bool few = rows_n <= 4 * kPrepareTokens;
         const int prepare_tokens = few ? kPrepareFew : kPrepareTokens;
-        L(KC_PREPARE_LINEAR, few ? k_bprepare<128, kPrepareFew> : k_bprepare<128, kPrepareTokens>,
-          dim3((unsigned)((d.QKV + 127) / 128), (unsigned)((rows_n + prepare_tokens - 1) / prepare_tokens)), dim3(kBlock), 0,
+        L(KC_PREPARE_LINEAR, few ? k_bprepare<kPrepareFew> : k_bprepare<kPrepareTokens>,
+          dim3((unsigned)((d.QKV + kBKeyDim - 1) / kBKeyDim), (unsigned)((rows_n + prepare_tokens - 1) / prepare_tokens)), dim3(kBlock), 0,
           (const uint16_t*)qkv, (const uint16_t*)s->cache, conv_base, params, first, rows_n,
           (const float*)W(9), (int)d.QKV, c.key_heads, conv, qn, kn);
         L(KC_PREPARE_LINEAR, k_bhistory, dim3(grid_for((3 * d.QKV + kBlock - 1) / kBlock, 1024)),
           dim3(kBlock), 0, (const uint16_t*)qkv, rows_n, s->cache, conv_base, params, first,
           (int)d.QKV);
         const float scale = 1.0f / sqrtf((float)c.key_dim);  // DELTA_SCALE_BITS, qwen35.rs:703
-        auto scan = k_bscan<4>;  // key elements per lane: key_dim / 32
-        if (c.key_dim == 32) scan = k_bscan<1>;
-        else if (c.key_dim == 64) scan = k_bscan<2>;
-        else if (c.key_dim == 256) scan = k_bscan<8>;
-        L(KC_DELTA, scan, dim3((unsigned)(d.VS / 8)), dim3(kBlock), bscan_lds_bytes(c.key_dim),
+        L(KC_DELTA, k_bscan, dim3((unsigned)(d.VS / 8)), dim3(kBlock), kScanLds,
           (const uint16_t*)conv, (const uint16_t*)qn, (const uint16_t*)kn, (const uint16_t*)alpha,
           (const uint16_t*)beta, (const float*)W(5), (const float*)W(6), s->shadow + l * d.REC,
           rows_n, (int)d.VS, c.value_dim, VH, c.key_heads, (int)d.QKV, scale, core);
@@ -2229,7 +2221,7 @@ extern "C" int cq35_step(cq35_session* s, const uint64_t* tokens, int64_t n, int
       return fail(CQ35_ERANGE, "token prefix contains an ID outside the %d-token vocabulary", c.vocab);
   // Multi-token calls at key_dim 128 take the batched prefill
   // (text-dispatch, prefill.rs:623-652); smaller key dims fold token by token.
-  const bool batched = n >= 2 && c.key_dim == 128;
+  const bool batched = n >= 2 && c.key_dim == kBKeyDim;
   if (batched) {
     if (const char* why = prefill_unsupported(*s->model))
       return fail(CQ35_EUNSUPPORTED, "batched prefill: %s", why);

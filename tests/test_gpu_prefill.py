@@ -2,8 +2,9 @@
 text-batch, src/qwen/prefill.rs:36-653) against the CPU restatement on an
 MI355X: greedy token, BF16 logits and the whole session state bit-exact after
 the batched call and over the decode steps that follow it, for a dense and a
-MoE shape, calls spanning two 1024-token chunks (dense and MoE), and a call
-that starts after earlier tokens (convolution taps from the cache history)."""
+MoE shape, calls spanning two chunks (dense and MoE; 256 rows, as where
+memory is short, and the usual 1024), and a call that starts after earlier
+tokens (convolution taps from the cache history)."""
 import numpy as np
 import pytest
 
@@ -77,16 +78,18 @@ def test_batched_prefill_after_decoded_tokens(oracle):
     run(oracle, "mini-moe", 15, before, prompt, 4)
 
 
-def test_batched_prefill_two_chunks(oracle):
+def test_batched_prefill_two_chunks(oracle, monkeypatch):
+    monkeypatch.setenv("CQ35_PREFILL_ROWS", "256")
     cfg = cc.preset("mini")
     prompt = np.random.default_rng(53).integers(0, cfg["vocab"], 300).tolist()
     run(oracle, "mini", 16, [], prompt, 3)
 
 
-def test_batched_prefill_two_chunks_moe(oracle):
-    """300 MoE tokens: about 75 tokens are routed to each of mini-moe's 32
-    experts, so the grouped gate/up runs its per-lane
+def test_batched_prefill_two_chunks_moe(oracle, monkeypatch):
+    """300 MoE tokens: the first 256-token chunk routes about 64 tokens to each
+    of mini-moe's 32 experts, so the grouped gate/up runs its per-lane
     epilogues across the 64-token boundary."""
+    monkeypatch.setenv("CQ35_PREFILL_ROWS", "256")
     cfg = cc.preset("mini-moe")
     prompt = np.random.default_rng(54).integers(0, cfg["vocab"], 300).tolist()
     run(oracle, "mini-moe", 17, [], prompt, 3)
