@@ -28,14 +28,20 @@
 // end, one output per thread, through LDS. Two visits of all rows are staged
 // per barrier with whole-line loads straight into LDS, three stages ahead.
 //
-// Bound: issue. The F32 matrix instructions run at 75 T multiply-adds/s on
-// this part and share the issue slots with the vector unit (16 operand
-// extractions per 12 of them alone bring them to 58, the tree adds further):
-// 12352 rows x 2048 columns x 768 tokens take 653 us, 29.8 T/s; 2048 x 6144
-// 279 us, 34.7 T/s. With all loads taken out the first is 8 % faster, so wider
-// tiles (48 x 16 is what the registers hold: 64 sums of three levels) or
-// another load path gain little. The vector kernel (k_bproject) reached 11
-// T/s: eight 2B layers of a 777-token prompt went from 43.4 to 20.4 ms.
+// Bound: no one unit. The F32 matrix instructions alone run at 75 T
+// multiply-adds/s on this part; 12352 rows x 2048 columns x 768 tokens take 653
+// us, 29.8 T/s, 2048 x 6144 279 us, 34.7 T/s. Counters of the plain 48 x 16
+// form (2B layers, 777 tokens): the matrix cores are busy 40 % of a SIMD's
+// cycles (46 % in the residual form), other vector instructions (4.4 per
+// matrix instruction: operands, tree adds, addresses) issue in 22 %, and for
+// the rest neither: a SIMD's two waves are in the same stage, with a barrier
+// per 12 matrix instructions, and spend 27 % of their time in waits and 44 %
+// with an instruction ready that the unit is not free for. LDS is active 22 %
+// of the time, three tenths of that conflicts; with all loads
+// taken out the kernel is 8 % faster. Wider tiles (48 x 16 is what the
+// registers hold: 64 sums of three levels) gain little. The vector kernel
+// (k_bproject) reached 11 T/s: eight 2B layers of a 777-token prompt went from
+// 43.4 to 20.4 ms.
 #pragma once
 
 #include "prefill.h"

@@ -246,6 +246,26 @@ def test_products_alone(kind, mode, n):
         assert np.array_equal(got[~nan], want[~nan]), (kernel, int((got[~nan] != want[~nan]).sum()))
 
 
+@pytest.mark.parametrize("mode, n, rows", [(0, 777, 5001), (1, 300, 2050), (2, 777, 3100), (2, 20, 1100)])
+def test_every_region_recomputed(mode, n, rows):
+    """Whole matrices of products that the matrix cores round differently: more
+    row groups than the recomputation has groups of waves, more than one batch
+    of 64 regions each, ragged ends. Against the vector kernel, bit for bit."""
+    cols = 512
+    print("every region, mode", mode, "tokens", n, "rows", rows, flush=True)
+    rng = np.random.default_rng(rows)
+    x = operands("tiny", 0, n, 32, cols, rng)[0]
+    m = rng.integers(32, 64, (rows, cols)) * 4
+    small = narrow((np.where(rng.random(m.shape) < 0.5, m + 1, -(m + 3)) * 2.0 ** -79).astype(np.float32))
+    plain = narrow(rng.standard_normal((rows, cols)).astype(np.float32) * np.float32(2.0 ** 60))
+    res = narrow((rng.integers(-64, 64, (n, rows)) * 2.0 ** -132).astype(np.float32)) if mode == 1 else None
+    w, w2 = (plain, small) if mode == 2 else (small, None)
+    few = slice(0, 64)
+    assert (narrow(b256(x[:20], small[few], True)) != narrow(b256(x[:20], small[few]))).mean() > 0.001
+    want, got = exact_gemm(x, w, w2, res, mode, 0), exact_gemm(x, w, w2, res, mode, 1)
+    assert np.array_equal(want, got), int((want != got).sum())
+
+
 def test_numpy_order_is_the_restatement(oracle):
     rng = np.random.default_rng(9)
     for kind in ("ordinary", "cancelling", "subnormal sums", "tiny", "huge"):
