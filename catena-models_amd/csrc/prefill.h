@@ -371,8 +371,8 @@ __device__ __forceinline__ float sum32_everywhere(float v) {
 // and rate (the next stage's rows are requested before the chain starts); a
 // token's values are read from LDS a token ahead; the sums leave their total
 // in every lane; lane t keeps token t's output, and scale, rounding and store
-// run once per stage: 67 vector instructions a token. 1024 tokens of a 35B
-// layer take 225 us (355 with BF16 rows widened and the totals broadcast
+// run once per stage: 67 vector instructions a token. 2048 tokens of a 35B
+// layer take 443 us; 1024 of them 225 before the gates went first (355 with BF16 rows widened and the totals broadcast
 // inside the chain; 16 lanes per channel, a quarter fewer instructions but one
 // wave per SIMD: 218).
 constexpr int kScanTokens = 32;
@@ -423,7 +423,14 @@ __global__ __launch_bounds__(kBlock) void k_bscan(
     al = alpha[(size_t)t * value_heads + head];
     be = beta[(size_t)t * value_heads + head];
   };
+  // the gates' chain of the first wave ahead of the rows that all widen (443
+  // against 456 us per 2048 tokens of a 35B layer the other way round)
   auto place = [&]() {
+    sval[threadIdx.x] = bf2f(val);
+    if (threadIdx.x < kScanTokens) {
+      const float time_step = softplus(bf2f(al) + dth);
+      sgate[threadIdx.x] = float2{hexp(rbf(time_step * ah)), rbf(sigmoid(bf2f(be)))};
+    }
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
       const int idx = threadIdx.x + kBlock * r;
@@ -434,11 +441,6 @@ __global__ __launch_bounds__(kBlock) void k_bscan(
       };
       widen(sk, kq4[r]);
       widen(sq, qq4[r]);
-    }
-    sval[threadIdx.x] = bf2f(val);
-    if (threadIdx.x < kScanTokens) {
-      const float time_step = softplus(bf2f(al) + dth);
-      sgate[threadIdx.x] = float2{hexp(rbf(time_step * ah)), rbf(sigmoid(bf2f(be)))};
     }
   };
   struct Token {
