@@ -372,9 +372,9 @@ __device__ __forceinline__ float sum32_everywhere(float v) {
 // token's values are read from LDS a token ahead; the sums leave their total
 // in every lane; lane t keeps token t's output, and scale, rounding and store
 // run once per stage: 67 vector instructions a token. 2048 tokens of a 35B
-// layer take 443 us; 1024 of them 225 before the gates went first (355 with BF16 rows widened and the totals broadcast
-// inside the chain; 16 lanes per channel, a quarter fewer instructions but one
-// wave per SIMD: 218).
+// layer take 443 us; 1024 of them 225 before the gates went first (355 with
+// BF16 rows widened and the totals broadcast inside the chain; 16 lanes per
+// channel, a quarter fewer instructions but one wave per SIMD: 218).
 constexpr int kScanTokens = 32;
 
 constexpr size_t kScanLds = (size_t)kScanTokens * kBKeyDim * 2 * 4 + (size_t)kScanTokens * 8 + (size_t)kScanTokens * 8 * (4 + 2);

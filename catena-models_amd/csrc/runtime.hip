@@ -76,13 +76,14 @@ BlockPool<HipMemory>& device_pool(int device) {
 // hipMalloc on the current device; its idle chunk buffers make way.
 template <typename T>
 hipError_t device_malloc(T** p, size_t bytes) {
-  hipError_t e = hipMalloc((void**)p, bytes);
+  const hipError_t e = hipMalloc((void**)p, bytes);
+  if (e == hipSuccess) return e;
+  hipGetLastError();  // returned here, not at the next launch
   int device = 0;
-  if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && device_pool(device).trim()) {
-    hipGetLastError();
-    e = hipMalloc((void**)p, bytes);
-  }
-  return e;
+  if (e != hipErrorOutOfMemory || hipGetDevice(&device) != hipSuccess || !device_pool(device).trim()) return e;
+  const hipError_t again = hipMalloc((void**)p, bytes);
+  if (again != hipSuccess) hipGetLastError();
+  return again;
 }
 
 }  // namespace
@@ -1606,24 +1607,18 @@ int prefill_buffers(PrefillLease* lease) {
   cq35_session* s = lease->s;
   const int64_t limit = s->prefill_rows ? s->prefill_rows : s->matrix ? kMChunk : kBChunk;
   const int64_t room = (s->capacity + 15) / 16 * 16;
-  const int64_t rows = std::min(limit, room), few = std::min(s->matrix ? kMFewRows : kBFewRows, rows);
-  auto& pool = device_pool(s->model->device);
-  auto bytes = [&](int64_t m) {
+  long rows = std::min(limit, room);
+  const long few = std::min<long>(s->matrix ? kMFewRows : kBFewRows, rows);
+  auto bytes = [&](long m) {
     Prefill pf;
     return prefill_layout(s, m, nullptr, &pf);
   };
-  int64_t m = rows;
-  lease->block = pool.idle(bytes(m));
-  if (!lease->block.p) {
+  lease->block = lend_rows(device_pool(s->model->device), &rows, few, bytes, [] {
     size_t free_bytes = 0, total_bytes = 0;
-    HIP_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
-    if (bytes(m) > free_bytes / 8) m = few;
-    if (m < rows) lease->block = pool.idle(bytes(m));
-    if (!lease->block.p) lease->block = pool.allocate(bytes(m));
-    if (!lease->block.p && m > few) lease->block = pool.allocate(bytes(m = few));
-    if (!lease->block.p) return fail(CQ35_EDEVICE, "no device memory for %zu bytes of prompt buffers", bytes(m));
-  }
-  prefill_layout(s, m, static_cast<unsigned char*>(lease->block.p), &lease->pf);
+    return hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess ? free_bytes : (size_t)0;
+  });
+  if (!lease->block.p) return fail(CQ35_EDEVICE, "no device memory for %zu bytes of prompt buffers", bytes(rows));
+  prefill_layout(s, rows, static_cast<unsigned char*>(lease->block.p), &lease->pf);
   return CQ35_OK;
 }
 

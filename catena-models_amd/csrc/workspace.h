@@ -103,4 +103,20 @@ class BlockPool {
   int users_ = 0;
 };
 
+// A block of `pool` for *rows rows of bytes(rows), or for `few` of them where
+// a new block would take an eighth of the free memory or is not to be had;
+// *rows what it became. free_bytes() is asked for new blocks only.
+template <typename Pool, typename Bytes, typename Free>
+DeviceBlock lend_rows(Pool& pool, long* rows, long few, Bytes bytes, Free free_bytes) {
+  DeviceBlock block = pool.idle(bytes(*rows));
+  if (block.p) return block;
+  if (bytes(*rows) > free_bytes() / 8 && few < *rows) {
+    *rows = few;
+    block = pool.idle(bytes(few));
+  }
+  if (!block.p) block = pool.allocate(bytes(*rows));
+  if (!block.p && few < *rows) block = pool.allocate(bytes(*rows = few));
+  return block;
+}
+
 }  // namespace cq35

@@ -2,7 +2,9 @@
 (catena-models_amd/csrc/workspace.h), compiled for the host over a counted
 allocator: blocks are lent again, a larger need replaces a smaller idle block,
 at most eight stay idle, a failed allocation takes the idle ones back first,
-the last model gives everything back, and threads never share a block."""
+the last model gives everything back, threads never share a block, and fewer
+rows are taken where a new block would take an eighth of the free memory or is
+not to be had."""
 import os
 import subprocess
 
@@ -80,6 +82,35 @@ int main(int, char** argv) {
     CHECK(blocks == 1);
     pool.give(out);  // no model left: not kept
     CHECK(blocks == 0);
+  } else if (!strcmp(argv[1], "rows")) {
+    size_t room = 1 << 20;
+    int asked = 0;
+    auto bytes = [](long m) { return (size_t)m * 10; };
+    auto room_left = [&] { return ++asked, room; };
+    long rows = 1000;
+    DeviceBlock b = lend_rows(pool, &rows, 200, bytes, room_left);
+    CHECK(rows == 1000 && b.bytes == 10000 && asked == 1);
+    pool.give(b);
+    room = 79999;  // an eighth is less than a block of 1000 rows: an idle one will do, a new one not
+    b = lend_rows(pool, &rows, 200, bytes, room_left);
+    CHECK(rows == 1000 && asked == 1);
+    DeviceBlock c = lend_rows(pool, &rows, 200, bytes, room_left);
+    CHECK(rows == 200 && c.bytes == 2000 && asked == 2);
+    pool.give(b), pool.give(c);
+    b = lend_rows(pool, &(rows = 5000), 200, bytes, room_left);  // an idle block of more than the few rows
+    CHECK(rows == 200 && b.bytes == 2000);
+    pool.give(b);
+    room = 1 << 20;
+    limit = 30000;
+    b = lend_rows(pool, &(rows = 5000), 200, bytes, room_left);  // no such block to be had
+    CHECK(rows == 200 && b.p);
+    pool.give(b);
+    limit = 0;
+    CHECK(!lend_rows(pool, &(rows = 5000), 4000, bytes, room_left).p);
+    rows = 16;
+    limit = 1 << 20;
+    room = 0;
+    CHECK(lend_rows(pool, &rows, 16, bytes, room_left).p && rows == 16);
   } else {  // threads: a lent block is written and read by its holder alone
     std::atomic<int> wrong{0};
     std::vector<std::thread> threads;
@@ -113,7 +144,7 @@ def program(tmp_path_factory):
     return str(d / "pool")
 
 
-@pytest.mark.parametrize("what", ["again", "most", "short", "last", "threads"])
+@pytest.mark.parametrize("what", ["again", "most", "short", "last", "rows", "threads"])
 def test_pool(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
